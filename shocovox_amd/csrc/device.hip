@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256) void cast_kernel(TreeView t, const float* __re
 
 // get_by_ray_at_lod for a ray array (MIP bricks probed per the viewing
 // distance when the tree's MIPs are enabled).
-__global__ __launch_bounds__(256) void cast_lod_kernel(TreeView t, const float* __restrict__ rays,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void cast_lod_kernel(TreeView t, const float* __restrict__ rays,
                                                        uint32_t n, float viewing_distance,
                                                        const uint32_t* __restrict__ order,
                                                        HitPtrs out) {
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) void cast_lod_kernel(TreeView t, const float* 
 
 // get_by_ray_at_lod for the primary rays of a viewport: four 64-lane waves
 // per workgroup, each over one 8x8 pixel tile.
-__global__ __launch_bounds__(256) void render_lod_kernel(TreeView t, Camera cam, uint32_t w,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void render_lod_kernel(TreeView t, Camera cam, uint32_t w,
                                                          uint32_t h, float viewing_distance,
                                                          HitPtrs out) {
   const uint32_t lane = threadIdx.x & 63u;

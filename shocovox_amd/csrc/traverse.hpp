@@ -396,17 +396,53 @@ SVO_HD __attribute__((always_inline)) inline bool probe_brick(const TreeView& t,
 // the box's far corner or stays), so no later position passes the test and
 // the ray ends as a miss. Only the nudges and the iteration count remain,
 // replayed here exactly (the restart's interior test, then one counted
-// iteration per restart). Not for MIP-enabled LOD rays (their MIP test runs
-// on every iteration) nor for a leaf root (its brick probe does).
+// iteration per restart), and only when the count can decide anything: the
+// ray ends as a miss either way, so the nudges matter only if they could
+// exceed the iteration bound before p leaves the tree. A nudge moves p by
+// fl(p + s) - p with s = fl(0.1 d); for a result inside the tree the rounding
+// is at most size * 2^-25, so with m = max |s| >= size * 2^-20 every counted
+// nudge moves p by at least 31/32 m along that axis, always the same way, and
+// at most 1.04 size / m + 1 of them end inside the tree. When that is within
+// the iterations left (tested with a factor of two to spare) the result is
+// known at once. (A NaN component of s makes p leave at the first nudge.)
+// The replay is one chain of adds and compares per ray, thousands long in a
+// large tree: without it a 4K frame of a 1024^3 heightfield takes 0.72 ms
+// instead of 3.04 ms, 24 views of 12 small trees in one batched run 0.71 ms
+// instead of 1.29 ms, and a 720p LOD frame of a 256^3 heightfield 0.25 ms
+// instead of 2.72 ms.
+// Not for a leaf root (its brick probe runs on every iteration), nor for
+// MIP-enabled LOD rays unless mip_test_over holds.
 SVO_HD inline CastResult crawl_out_of_root(const TreeView& t, V3f p, V3f d, uint32_t steps,
                                            uint32_t flags) {
+  const V3f s = d * 0.1f;
+  const float m = fmaxf(fmaxf(fabsf(s.x), fabsf(s.y)), fabsf(s.z));
+  const uint32_t left = t.max_steps - steps;  // (no ray gets here past its bound)
+  if (left >= 16u && m >= t.size * 0x1p-20f && m * static_cast<float>(left) >= 2.0f * t.size)
+    return miss_flags(flags);
   for (;;) {
-    p = p + d * 0.1f;
+    p = p + s;
     if (!((p.x < t.size) & (p.y < t.size) & (p.z < t.size) & (p.x > 0.0f) & (p.y > 0.0f) &
           (p.z > 0.0f)))
       return miss_flags(flags);
     if (++steps > t.max_steps) return miss_flags(flags | FLAG_ITERATION_GUARD);
   }
+}
+
+// Whether the MIP test at the root (level < |o - snapped| / viewing distance,
+// snapped being p rounded to a grid of 2 level) fails now and in every later
+// restart of a ray that crawls out of the root. The level rises by one per
+// restart and never falls; snapped lies within level of p per axis, so
+// |o - snapped| <= far + 1.7321 level, far being the distance from o to the
+// tree's farthest corner (0.1% covers the roundings of both sides). Once
+// level * (viewing distance - 1.75) >= 1.001 far holds it holds from then on
+// (for a viewing distance above 1.75).
+SVO_HD inline bool mip_test_over(const TreeView& t, V3f o, float mip_level,
+                                 float viewing_distance) {
+  const V3f far{fmaxf(fabsf(o.x), fabsf(o.x - t.size)), fmaxf(fabsf(o.y), fabsf(o.y - t.size)),
+                fmaxf(fabsf(o.z), fabsf(o.z - t.size))};
+  const float f = 1.001f * length(far);  // (infinite: |o - snapped| may be, too)
+  return viewing_distance > 1.75f && f < __builtin_inff() &&
+         mip_level * (viewing_distance - 1.75f) >= f;
 }
 
 // The reference's NodeStack<u32, 4> (raytracing_on_cpu.rs:19-82): a ring of
@@ -481,6 +517,7 @@ SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
   }
   if (target == OOB_OCTANT) return miss_flags(0u);
   uint32_t steps = 0;
+  bool crawl = false;  // LOD: the ray ends in crawl_out_of_root, after the loop
   // log2(size / dim) of two powers of two, exactly
   float mip_level =
       LOD ? static_cast<float>(__builtin_ctz(static_cast<uint32_t>(t.size) / t.dim)) : 0.0f;
@@ -573,8 +610,15 @@ SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
       if (!pop || stk.count > 1u) st = dda_step(d, sig, &p, pop ? bounds : tb, scale);
       if (pop) {
         if (stk.count == 1u && key == 0u && !backtrack && target != OOB_OCTANT &&
-            kind != KIND_LEAF && !(LOD && t.mips_enabled))
-          return crawl_out_of_root(t, p, d, steps, r.flags);
+            kind != KIND_LEAF &&
+            (!LOD || !t.mips_enabled || n.mip == FORM_EMPTY ||
+             mip_test_over(t, o, mip_level, viewing_distance))) {
+          // (in place here, after the loop there: the faster of the two in
+          // either build, by 2% and 1%)
+          if constexpr (!LOD) return crawl_out_of_root(t, p, d, steps, r.flags);
+          crawl = true;
+          break;
+        }
         if (stk.count > 1u) {
           // the parent's bounds and the sibling the step leads to
           const float s2 = bounds.size * 2.0f;
@@ -641,6 +685,8 @@ SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
     bounds = next_bounds;
     target = next_target;
   }
+  if constexpr (LOD)
+    if (crawl) return crawl_out_of_root(t, p, d, steps, r.flags);
   return miss_flags(r.flags);
 hit_found:
   r.hit = 1;

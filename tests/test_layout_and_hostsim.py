@@ -362,6 +362,31 @@ def test_rays_that_leave_the_content_behind():
                 assert g1.tobytes() == g2.tobytes(), (size, limit, form)
 
 
+@pytest.mark.parametrize("scale", [1.0, 3e-4, 1e-6, 1e6, float("inf")])
+def test_crawl_result_without_its_nudges(scale):
+    """crawl_out_of_root knows its result without replaying the nudges when
+    they cannot exceed the iteration bound: bounds below, around and far above
+    the number of nudges, and directions of any length, give the result of the
+    restarts run one by one."""
+    for tree in (Octree.new(64, 4), Octree.scene(1, 128, 8, 3)):
+        size = tree.get_size()
+        a = tree.flatten().arrays()
+        rays = W.incoherent_rays(size, 300, seed=11)
+        with np.errstate(invalid="ignore"):
+            rays[:, 3:] *= np.float32(scale)
+        rays[0, 3:] = (0.0, 0.0, 1.0)  # axis-aligned: the other axes do not move
+        rays[1, 3:] = (1e-30, 0.0, -1e-30)
+        rays[2, 4] = np.nan
+        flags = []
+        for limit in (15, 16, 17, 2 * size, 10 * size, 20 * size, 40 * size):
+            base = hostsim.cast(a, rays, max_steps=limit, regrouped="nocrawl")
+            for form in (False, True):
+                got = hostsim.cast(a, rays, max_steps=limit, regrouped=form)
+                assert base.tobytes() == got.tobytes(), (size, limit, form)
+            flags.append(int((base["flags"] & 1).sum()))
+        assert scale > 1.0 or flags[0] > 0  # some rays meet the lowest bound
+
+
 def test_regrouped_traversal_under_forced_guard():
     """cast_ray_ww counts iterations exactly as cast_ray (an iteration
     resumed after its probe is not counted twice): with lowered bounds both

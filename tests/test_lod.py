@@ -140,3 +140,26 @@ def test_edited_mips_reach_the_mirror():
         assert canonical_layout(flat.arrays()) == canonical_layout(t.flatten().arrays())
         got = hostsim.cast(flat.arrays(), rays, viewing_distance=3.0)
         assert_parity(_oracle(t).cast(rays, viewing_distance=3.0), got, f"round {rnd}")
+
+
+@pytest.mark.parametrize("vd", [0.5, 1.75, 1.8, 5.0, 64.0, 1e6, F32_MAX])
+def test_lod_rays_that_leave_the_content_behind(vd):
+    """LOD rays with nothing ahead of them at the root end without replaying
+    their restarts once the MIP test can no longer pass (mip_test_over): same
+    results as the oracle, which runs them all, from eyes near and far."""
+    t = Octree.new(64, 4)
+    rng = np.random.default_rng(8)
+    xyz = rng.integers(0, 12, size=(300, 3)).astype(np.uint32)
+    ents = np.zeros((300, 3), np.uint32)
+    ents[:, 0] = 1
+    ents[:, 1] = (rng.integers(1, 250, size=300).astype(np.uint32) << 24) | 0xFF
+    t.insert_many(xyz, ents)
+    t.albedo_mip_map_resampling_strategy().switch_albedo_mip_maps(True).recalculate_mips()
+    f = t.flatten().arrays()
+    rays = W.incoherent_rays(64, 500, seed=4)
+    far = rays[:200].copy()
+    far[:, :3] -= far[:, 3:] * np.float32(3000.0)
+    far[0, :3] = 1e30
+    rays = np.concatenate([rays, far])
+    assert_parity(_oracle(t).cast(rays, viewing_distance=vd),
+                  hostsim.cast(f, rays, viewing_distance=vd), f"vd={vd}")
