@@ -295,17 +295,15 @@ SVO_HD __attribute__((always_inline)) inline bool probe_brick(const TreeView& t,
       return static_cast<uint32_t>(x + y * dim + z * dim * dim);
     }
   };
-  // The loop has one exit: the cell is outside the brick, or occupied, or
-  // (without P2) the step bound is reached (then `in` still holds and
-  // `occupied` not). The occupancy word is read for every cell, from index 0
-  // when the cell is outside, so that the test needs no branch.
+  // After the loop `occupied` says whether the ray stands in an occupied cell,
+  // `in` (when not) whether it stopped inside the brick: on a NaN step or,
+  // without P2, at the step bound.
   bool in, occupied;
   if constexpr (P2) {
     // Cell coordinates mirrored on the axes whose signum is -1: a = ix
     // (signum +1) or dim-1-ix = ix ^ (dim-1) (signum -1), so that every move
     // is +1 and an axis leaves the brick at a = dim; the cell's flat index is
-    // the mirrored one xor the mirror mask. With dim a power of two, all
-    // three are below dim exactly when their bitwise or is.
+    // the mirrored one xor the mirror mask.
     const uint32_t dm1 = t.dim - 1u;
     const uint32_t nx = sig.x < 0.0f ? dm1 : 0u;
     const uint32_t ny = sig.y < 0.0f ? dm1 : 0u;
@@ -327,29 +325,59 @@ SVO_HD __attribute__((always_inline)) inline bool probe_brick(const TreeView& t,
                   bb.min.y),
              fmaf(static_cast<float>(static_cast<uint32_t>(iz) + (sig.z < 0.0f ? 0u : 1u)), unit,
                   bb.min.z)};
+    // Each iteration takes the step out of the current cell while the cell's
+    // word is still in flight, requests the next cell's word, and only then
+    // keeps the step or, when the cell was occupied, drops it (by selects on
+    // p and the index; the other state is not used after the loop). So a step
+    // waits for its load only as long as its own arithmetic does not cover
+    // it, and the loop has one exit and no masks to carry: a lone ray's step
+    // 450 -> 275 cycles (the loop is 41 VALU + 8 SALU, where testing the cell
+    // before stepping was 31 VALU + 27 SALU), 8 1080p frames in one batched
+    // run 1.09 -> 0.97 ms.
+    uint32_t flat = (ax | (ay << shift) | (az << (2u * shift))) ^ mirror;
+    uint32_t bits = occ_word(t, occ_off, flat, true);
+    uint32_t bit;
+    float m;
     for (;;) {
-      in = (ax | ay | az) < t.dim;
-      const uint32_t flat = (ax | (ay << shift) | (az << (2u * shift))) ^ mirror;
-      const uint32_t bits = occ_word(t, occ_off, flat, in);
-      occupied = in & (bit_of(bits, flat) != 0u);
-      if (!in | occupied) break;
       bool sx, sy, sz;
-      const float m = dda_step_far(d, p, cmin, scale, &sx, &sy, &sz);
+      V3f q = *p;
+      m = dda_step_far(d, &q, cmin, scale, &sx, &sy, &sz);
       cmin = V3f{sx ? cmin.x + umove.x : cmin.x, sy ? cmin.y + umove.y : cmin.y,
                  sz ? cmin.z + umove.z : cmin.z};
       ax += static_cast<uint32_t>(sx);
       ay += static_cast<uint32_t>(sy);
       az += static_cast<uint32_t>(sz);
-      // A step of length m (not NaN) moves at least one axis, each axis only
-      // in its direction's sign (signum is +-1 there: a NaN direction makes
-      // every distance NaN), so the cell leaves the brick within 3 dim
-      // steps. A NaN step moves nothing (p becomes NaN and stays so), so the
-      // loop would repeat that state: it ends here.
-      if (!(m == m)) break;
+#if defined(__HIP_DEVICE_COMPILE__)
+      // (the word is read from here on, behind the step's arithmetic)
+      asm volatile("" : "+v"(bits) : "v"(ax), "v"(ay), "v"(az));
+#endif
+      bit = bit_of(bits, flat);
+      const bool keep = bit == 0u;
+      const uint32_t next = (ax | (ay << shift) | (az << (2u * shift))) ^ mirror;
+      const uint32_t axes = ax | ay | az;
+      bits = occ_word(t, occ_off, next, axes < t.dim);
+      *p = V3f{keep ? q.x : p->x, keep ? q.y : p->y, keep ? q.z : p->z};
+      flat = keep ? next : flat;
+      // Leaves at an occupied cell, or outside the brick (an axis at dim: with
+      // dim a power of two, a bit of `axes` above dim - 1). A step of length m
+      // (not NaN) moves at least one axis, each axis only in its direction's
+      // sign (signum is +-1 there: a NaN direction makes every distance NaN),
+      // so the cell leaves the brick within 3 dim steps. A NaN step moves
+      // nothing (p becomes NaN and stays so), so the loop would repeat that
+      // state: it ends here.
+      const uint32_t stop = bit | (axes & ~dm1);
+      if ((stop != 0u) | !(m == m)) break;
     }
-    ix = static_cast<int>(ax ^ nx);
-    iy = static_cast<int>(ay ^ ny);
-    iz = static_cast<int>(az ^ nz);
+#if defined(__HIP_DEVICE_COMPILE__)
+    // (opaque here, so that the two tests below are made after the loop and
+    // not carried through it as masks)
+    asm volatile("" : "+v"(bit), "+v"(m));
+#endif
+    occupied = bit != 0u;
+    in = !(m == m);
+    ix = static_cast<int>(flat & dm1);
+    iy = static_cast<int>((flat >> shift) & dm1);
+    iz = static_cast<int>(flat >> (2u * shift));
   } else {
     V3f cmin = bb.min + V3f{static_cast<float>(ix), static_cast<float>(iy),
                             static_cast<float>(iz)} *
