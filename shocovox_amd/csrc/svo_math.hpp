@@ -164,6 +164,19 @@ SVO_HD inline uint32_t step_octant(uint32_t octant, V3f step) {
   return step_octant_signs(octant, step_int(step.x), step_int(step.y), step_int(step.z));
 }
 
+// Octant bits of three per-axis flags.
+SVO_HD inline uint32_t octant_of(bool x, bool y, bool z) {
+  return (x ? 1u : 0u) | (z ? 2u : 0u) | (y ? 4u : 0u);
+}
+
+// step_octant for a step along the axes of `moved` (octant bits) of a ray
+// that runs backwards along the axes of `neg`: an axis steps to the other
+// half, or out of the node when the half it is in is already the one the ray
+// runs towards (octant bit 1 forwards, 0 backwards).
+SVO_HD inline uint32_t step_octant_moved(uint32_t octant, uint32_t moved, uint32_t neg) {
+  return ((octant ^ neg) & moved) != 0u ? OOB_OCTANT : octant ^ moved;
+}
+
 // Cube{min_position, size}  (spatial/mod.rs:31-53)
 struct Cube {
   V3f min;

@@ -206,12 +206,10 @@ SVO_HD inline uint32_t bitmap_index(V3f bp, uint32_t* flags) {
   uint32_t x = f2u32(bp.x);
   uint32_t y = f2u32(bp.y);
   uint32_t z = f2u32(bp.z);
-  if (x > 3 || y > 3 || z > 3) {
-    *flags |= FLAG_BITMAP_RANGE;
-    x = x > 3 ? 3 : x;
-    y = y > 3 ? 3 : y;
-    z = z > 3 ? 3 : z;
-  }
+  *flags |= (x | y | z) > 3u ? FLAG_BITMAP_RANGE : 0u;
+  x = x > 3 ? 3 : x;
+  y = y > 3 ? 3 : y;
+  z = z > 3 ? 3 : z;
   return x + 4u * y + 16u * z;
 }
 
@@ -248,19 +246,14 @@ SVO_HD inline uint32_t bitmap_cell(V3f bp) {
   return clamp03(f2i32(bp.x)) + 4u * clamp03(f2i32(bp.y)) + 16u * clamp03(f2i32(bp.z));
 }
 
-// probe_brick (raytracing_on_cpu.rs:256-312) with traverse_brick (:156-252)
+// traverse_brick (raytracing_on_cpu.rs:156-252) over the occupancy of Parted
+// brick `word` with bounds bb: moves p to where the walk ends and returns
+// whether that is in an occupied cell, whose flat index goes to *cell.
 template <bool P2>
-SVO_HD __attribute__((always_inline)) inline bool probe_brick(const TreeView& t, uint32_t form,
-                                                              uint32_t word, Cube bb, V3f d,
-                                                              V3f sig, V3f scale, V3f* p,
-                                                              CastResult* r) {
-  if (form == FORM_EMPTY) return false;
-  if (form == FORM_SOLID) {
-    r->pix = word;
-    r->impact = *p;
-    r->cell = bb;
-    return true;
-  }
+SVO_HD __attribute__((always_inline)) inline bool walk_brick(const TreeView& t, uint32_t word,
+                                                             Cube bb, V3f d, V3f sig, V3f scale,
+                                                             V3f* p, uint32_t* cell,
+                                                             uint32_t* flags) {
   const int dim = static_cast<int>(t.dim);
   const float fdim = static_cast<float>(t.dim);
   const float rcp_size = size_rcp<P2>(bb.size);
@@ -401,19 +394,62 @@ SVO_HD __attribute__((always_inline)) inline bool probe_brick(const TreeView& t,
     }
   }
   if (occupied) {
-    const uint64_t n3 = static_cast<uint64_t>(t.dim) * t.dim * t.dim;
-    r->pix = t.brick_pix[static_cast<uint64_t>(word) * n3 + flat_of(ix, iy, iz)];
-    const V3f scaled = V3f{static_cast<float>(ix), static_cast<float>(iy),
-                           static_cast<float>(iz)} *
-                       bb.size;
-    const Cube hb{bb.min + div3_size<P2>(scaled, fdim, t.inv_dim),
-                  div_size<P2>(bb.size, fdim, t.inv_dim)};
-    r->impact = *p;
-    r->cell = hb;
+    *cell = flat_of(ix, iy, iz);
     return true;
   }
-  if (in) r->flags |= FLAG_ITERATION_GUARD;
+  if (in) *flags |= FLAG_ITERATION_GUARD;
   return false;
+}
+
+// The hit of a Solid brick, or of Parted brick `word` in flat cell `cell`, at p
+// (raytracing_on_cpu.rs:256-295).
+template <bool P2>
+SVO_HD __attribute__((always_inline)) inline void brick_hit(const TreeView& t, uint32_t form,
+                                                            uint32_t word, Cube bb,
+                                                            uint32_t cell, V3f p, CastResult* r) {
+  r->hit = 1;
+  r->impact = p;
+  if (form == FORM_SOLID) {
+    r->pix = word;
+    r->cell = bb;
+    return;
+  }
+  const float fdim = static_cast<float>(t.dim);
+  uint32_t ix, iy, iz;
+  if constexpr (P2) {
+    const uint32_t shift = static_cast<uint32_t>(__builtin_ctz(t.dim));
+    ix = cell & (t.dim - 1u);
+    iy = (cell >> shift) & (t.dim - 1u);
+    iz = cell >> (2u * shift);
+  } else {
+    ix = cell % t.dim;
+    iy = cell / t.dim % t.dim;
+    iz = cell / (t.dim * t.dim);
+  }
+  const uint64_t n3 = static_cast<uint64_t>(t.dim) * t.dim * t.dim;
+  r->pix = t.brick_pix[static_cast<uint64_t>(word) * n3 + cell];
+  // (below the brick dimension: exact as signed or unsigned)
+  const V3f scaled = V3f{static_cast<float>(static_cast<int>(ix)),
+                         static_cast<float>(static_cast<int>(iy)),
+                         static_cast<float>(static_cast<int>(iz))} *
+                     bb.size;
+  r->cell = Cube{bb.min + div3_size<P2>(scaled, fdim, t.inv_dim),
+                 div_size<P2>(bb.size, fdim, t.inv_dim)};
+}
+
+// probe_brick (raytracing_on_cpu.rs:256-312)
+template <bool P2>
+SVO_HD __attribute__((always_inline)) inline bool probe_brick(const TreeView& t, uint32_t form,
+                                                              uint32_t word, Cube bb, V3f d,
+                                                              V3f sig, V3f scale, V3f* p,
+                                                              CastResult* r) {
+  uint32_t cell = 0u;
+  if (form == FORM_EMPTY) return false;
+  if (form != FORM_SOLID &&
+      !walk_brick<P2>(t, word, bb, d, sig, scale, p, &cell, &r->flags))
+    return false;
+  brick_hit<P2>(t, form, word, bb, cell, *p, r);
+  return true;
 }
 
 // The rest of a ray whose POP of the root empties the stack because the
@@ -511,19 +547,37 @@ struct RingStack {
 // POP and is not reset by a restart from the root; when the level is below
 // |origin - round(p / (2 level)) * 2 level| / viewing_distance, the node's
 // MIP brick is probed over the node's bounds like a uniform leaf's brick.
+//
+// How a wave runs it. A ray's time is the latency of its iterations, and a
+// wave's the instructions of all paths its lanes take, so
+//   * the loop has one exit, on a status each lane keeps in a register;
+//     leaving from several places would carry a mask per place through every
+//     iteration (scalar instructions were a third of the loop's);
+//   * a hit lane leaves p, bounds, target and the stack as they are, and its
+//     palette value and cell are worked out after the loop, once per wave
+//     rather than in every iteration in which some lane hits (and the loop
+//     holds none of the result's registers: 63 VGPRs, where it held 77);
+//   * the LUT word of p's cell is requested beside the node record, not after
+//     the record has shown that it is needed; a probe that moved p requests
+//     it again;
+//   * a step is kept as octant bits (step_octant_moved).
+// Together a lone ray's iteration takes 0.56 us instead of 0.78, 8 1080p
+// frames in one batched run 0.90 ms instead of 0.96, one of them 0.185 ms
+// instead of 0.208.
 template <bool LOD, bool P2, class LutT>
 SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
     const TreeView& t, const LutT* __restrict__ lut, V3f o, V3f d, const NodeRec* top,
     uint32_t ntop, float viewing_distance) {
-  // Only the flags live across the loops; the probe fills pix, impact and
-  // cell on the hit path, and a miss returns miss_flags(flags). (Zeroing
-  // the hit fields up front would make the compiler carry them around every
-  // loop.)
   CastResult r;
+  r.hit = 0;
   r.flags = 0;
 
   const V3f scale = dda_scale_factors(d);
   const uint32_t dir_idx = hash_direction(d);
+  // the axes the ray runs backwards along (for a NaN component every scale
+  // factor is NaN and no step moves any axis)
+  const uint32_t neg =
+      octant_of(__builtin_signbit(d.x), __builtin_signbit(d.y), __builtin_signbit(d.z));
   const Cube root{v3u(0.0f), t.size};
   const float lo = 0.00001f;
   const float hi = 4.0f - 0.00001f;
@@ -545,14 +599,16 @@ SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
   }
   if (target == OOB_OCTANT) return miss_flags(0u);
   uint32_t steps = 0;
-  bool crawl = false;  // LOD: the ray ends in crawl_out_of_root, after the loop
+  uint32_t cell = 0;  // flat cell of a hit in a Parted brick
   // log2(size / dim) of two powers of two, exactly
   float mip_level =
       LOD ? static_cast<float>(__builtin_ctz(static_cast<uint32_t>(t.size) / t.dim)) : 0.0f;
+  enum : uint32_t { RUNS = 0, HIT = 1, HIT_MIP = 2, MISS = 3, GUARD = 4, CRAWL = 5 };
+  uint32_t end = RUNS;
   // One loop runs the reference's two: an iteration of its stack loop, and
-  // when the stack has emptied, first its restart from the root (which ends
-  // the ray when the nudged point leaves the tree).
-  for (;;) {
+  // when the stack has emptied, its restart from the root (which ends the ray
+  // when the nudged point leaves the tree).
+  do {
     // signum(d) per axis, formed again in every iteration from d's sign bits
     // (one instruction each) rather than kept in three registers: the empty
     // asm makes d opaque here, so the compiler cannot hoist these (or other
@@ -564,10 +620,7 @@ SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
     asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z));
 #endif
     V3f sig{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
-    if (++steps > t.max_steps) {
-      r.flags |= FLAG_ITERATION_GUARD;
-      break;
-    }
+    ++steps;  // (against the bound at the iteration's end)
     const uint32_t key = stk.s0;
     const NodeRec& n = (key < ntop ? top : t.nodes)[key];
     const uint64_t occ = n.occ;
@@ -576,148 +629,185 @@ SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
     // (same record, one round trip); with target OOB_OCTANT it is child[0]
     // and unused
     const uint32_t tword = n.child[target & 7u];
+    // the position in the node's 4x4x4 bitmap; the clamp to [lo, hi]
+    // (:425-436) is applied to the float position only where ADVANCE
+    // continues from it, the cell index comes from bitmap_cell
+    const float rcp_size = size_rcp<P2>(bounds.size);
+    V3f bp = bitmap_pos<P2>(p, bounds, rcp_size);
+    uint64_t ahead = lut[bitmap_cell(bp) * 8u + dir_idx];
+    auto moved_by_probe = [&]() {
+      bp = bitmap_pos<P2>(p, bounds, rcp_size);
+      ahead = lut[bitmap_cell(bp) * 8u + dir_idx];
+#if defined(__HIP_DEVICE_COMPILE__)
+      // (used here, so that the two requests are not merged into one after
+      // the probe)
+      asm volatile("" : "+v"(ahead));
+#endif
+    };
     const uint32_t kind = node_kind(meta);
-    bool backtrack = kind == KIND_UNIFORM_LEAF;
+    const bool uniform = kind == KIND_UNIFORM_LEAF;  // backtracks after its probe
     if (LOD && t.mips_enabled) {
       const float grid = mip_level * 2.0f;
       const V3f snapped{roundf(p.x / grid) * grid, roundf(p.y / grid) * grid,
                         roundf(p.z / grid) * grid};
-      if (mip_level < length(o - snapped) / viewing_distance &&
-          probe_brick<P2>(t, n.mip, n.mip_word, bounds, d, sig, scale, &p, &r))
-        goto hit_found;
+      if (mip_level < length(o - snapped) / viewing_distance) {
+        if (n.mip == FORM_SOLID) end = HIT_MIP;
+        if (n.mip == FORM_PARTED) {
+          if (walk_brick<P2>(t, n.mip_word, bounds, d, sig, scale, &p, &cell, &r.flags))
+            end = HIT_MIP;
+          moved_by_probe();
+        }
+      }
     }
-    if (target != OOB_OCTANT && (kind == KIND_UNIFORM_LEAF || kind == KIND_LEAF)) {
-      const bool uniform = kind == KIND_UNIFORM_LEAF;
+    if ((!LOD || end == RUNS) && target != OOB_OCTANT &&
+        (kind == KIND_UNIFORM_LEAF || kind == KIND_LEAF)) {
       const uint32_t slot = uniform ? 0u : target;
-      if (probe_brick<P2>(t, brick_form(meta, slot), slot == target ? tword : n.child[0],
-                          uniform ? bounds : child_bounds_for(bounds, target), d, sig, scale,
-                          &p, &r))
-        goto hit_found;
+      const uint32_t form = brick_form(meta, slot);
+      if (form == FORM_SOLID) end = HIT;
+      if (form == FORM_PARTED) {
+        if (walk_brick<P2>(t, slot == target ? tword : n.child[0],
+                           uniform ? bounds : child_bounds_for(bounds, target), d, sig, scale,
+                           &p, &cell, &r.flags))
+          end = HIT;
+        moved_by_probe();
+      }
     }
     // signum(d) formed again past the probe, so that the values formed
     // before it are dead inside the probe's DDA loop (whose registers then
     // hold the per-axis cell moves rather than recomputing them each step)
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z));
+    asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z), "+v"(end));
 #endif
-    sig = V3f{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
-    const float rcp_size = size_rcp<P2>(bounds.size);
-    // the position in the node's 4x4x4 bitmap; the clamp to [lo, hi]
-    // (:425-436) is applied to the float position only where ADVANCE
-    // continues from it, the cell index comes from bitmap_cell
-    V3f bp = bitmap_pos<P2>(p, bounds, rcp_size);
-    uint32_t flat = bitmap_cell(bp);
-    const bool pop = backtrack || target == OOB_OCTANT || occ == 0ull ||
-                     (occ & lut[flat * 8u + dir_idx]) == 0ull;
-    Cube tb = child_bounds_for(bounds, target);
-    // the child word is read only when the occupancy test passes (pure
-    // reads: the same decision as testing the child first)
-    const bool push = !pop && kind == KIND_INTERNAL &&
-                      (occ & octant_bitmap_mask(target)) != 0ull && tword != INVALID_INDEX;
-    // PUSH, POP and ADVANCE leave the next bounds and target here, and the
-    // stack moves once after them, by selects: the loop has a single back
-    // edge, so its state stays in the same registers on every path.
-    Cube next_bounds = bounds;
-    uint32_t next_target = target;
-    if (push) {
-      // PUSH (:484-492)
-      next_bounds = tb;
-      next_target = hash_region(p - tb.min, tb.size / 2.0f);
-    } else {
-      // POP (:445-475) and ADVANCE (:497-544) both begin with one DDA step,
-      // out of the node (POP, unless the stack empties) or out of the target
-      // child (ADVANCE); it is issued once for the lanes of both. (The POP's
-      // other values depend on the bounds only, so taking the step before
-      // them changes nothing.)
-      if (!pop && ++steps > t.max_steps) {
-        r.flags |= FLAG_ITERATION_GUARD;
-        break;
-      }
-      // (left unset when the POP empties the stack: then it is not read)
-      V3f st;
-      if (!pop || stk.count > 1u) st = dda_step(d, sig, &p, pop ? bounds : tb, scale);
-      if (pop) {
-        if (stk.count == 1u && key == 0u && !backtrack && target != OOB_OCTANT &&
-            kind != KIND_LEAF &&
-            (!LOD || !t.mips_enabled || n.mip == FORM_EMPTY ||
-             mip_test_over(t, o, mip_level, viewing_distance))) {
-          // (in place here, after the loop there: the faster of the two in
-          // either build, by 2% and 1%)
-          if constexpr (!LOD) return crawl_out_of_root(t, p, d, steps, r.flags);
-          crawl = true;
-          break;
-        }
-        if (stk.count > 1u) {
-          // the parent's bounds and the sibling the step leads to
-          const float s2 = bounds.size * 2.0f;
-          const float rcp_s2 = size_rcp<P2>(s2);
-          const V3f pmin{sub_fmod_size<P2>(bounds.min.x, s2, rcp_s2),
-                         sub_fmod_size<P2>(bounds.min.y, s2, rcp_s2),
-                         sub_fmod_size<P2>(bounds.min.z, s2, rcp_s2)};
-          const uint32_t from = pop_octant<P2>(bounds, pmin);
-          next_target = step_octant(from, st);
-          next_bounds = Cube{pmin, s2};
-        } else {
-          // the POP empties the stack: the reference's restart from the
-          // root (:551-562), which ends the ray once the nudged point has
-          // left the tree (taken here, not at the next iteration's start:
-          // nothing happens in between)
-          p = p + d * 0.1f;
-          next_target = ((p.x < t.size) & (p.y < t.size) & (p.z < t.size) & (p.x > 0.0f) &
-                         (p.y > 0.0f) & (p.z > 0.0f))
-                            ? hash_region(p, t.size / 2.0f)
-                            : OOB_OCTANT;
-          if (next_target == OOB_OCTANT) break;
-          next_bounds = root;
-        }
+    if (end == RUNS) {
+      sig = V3f{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
+      // (an empty bitmap has nothing ahead)
+      const bool pop = uniform | (target == OOB_OCTANT) | ((occ & ahead) == 0ull);
+      Cube tb = child_bounds_for(bounds, target);
+      const bool push = !pop & (kind == KIND_INTERNAL) &
+                        ((occ & octant_bitmap_mask(target)) != 0ull) & (tword != INVALID_INDEX);
+      const bool emptied = pop & (stk.count == 1u);
+      // PUSH, POP and ADVANCE leave the next bounds and target here, and the
+      // stack moves once after them, by selects: the loop's state stays in
+      // the same registers on every path.
+      Cube next_bounds = bounds;
+      uint32_t next_target = target;
+      if (push) {
+        // PUSH (:484-492)
+        next_bounds = tb;
+        next_target = hash_region(p - tb.min, tb.size / 2.0f);
       } else {
-        // the rest of ADVANCE
-        bool guard = false;
-        next_target = step_octant(target, st);
-        bp = V3f{rclamp(bp.x, lo, hi), rclamp(bp.y, lo, hi), rclamp(bp.z, lo, hi)};
-        while (next_target != OOB_OCTANT) {
-          tb = child_bounds_for(bounds, next_target);
-          bp = bp + bitmap_move<P2>(st, bounds.size, rcp_size);
-          flat = bitmap_index(bp, &r.flags);
-          // stop at a reachable occupied child or a non-empty leaf brick; the
-          // tests run cheapest first and the child word is read last
-          if (kind == KIND_LEAF && brick_form(meta, next_target) != FORM_EMPTY) break;
-          if (kind == KIND_INTERNAL && (occ & octant_bitmap_mask(next_target)) != 0ull &&
-              (lut[flat * 8u + dir_idx] & occ) != 0ull && n.child[next_target] != INVALID_INDEX)
-            break;
-          if (++steps > t.max_steps) {
-            guard = true;
-            break;
+        // POP (:445-475) and ADVANCE (:497-544) both begin with one DDA step,
+        // out of the node (POP, unless the stack empties) or out of the
+        // target child (ADVANCE); it is issued once for the lanes of both.
+        // (The POP's other values depend on the bounds only, so taking the
+        // step before them changes nothing; nor does a step taken by an
+        // ADVANCE that then meets the iteration bound, which ends the ray as
+        // a miss.)
+        bool sx = false, sy = false, sz = false;
+        if (!emptied)
+          dda_step_axes(d, sig, &p, (pop ? bounds : tb).min, (pop ? bounds : tb).size, scale, &sx,
+                        &sy, &sz);
+        const uint32_t moved = octant_of(sx, sy, sz);
+        if (pop) {
+          if (emptied) {
+            if (key == 0u && !uniform && target != OOB_OCTANT && kind != KIND_LEAF &&
+                (!LOD || !t.mips_enabled || n.mip == FORM_EMPTY ||
+                 mip_test_over(t, o, mip_level, viewing_distance))) {
+              end = CRAWL;
+            } else {
+              // the reference's restart from the root (:551-562), which ends
+              // the ray once the nudged point has left the tree (taken here,
+              // not at the next iteration's start: nothing happens in
+              // between)
+              p = p + d * 0.1f;
+              const bool inside = (p.x < t.size) & (p.y < t.size) & (p.z < t.size) &
+                                  (p.x > 0.0f) & (p.y > 0.0f) & (p.z > 0.0f);
+              next_target = hash_region(p, t.size / 2.0f);
+              next_bounds = root;
+              end = inside ? RUNS : MISS;
+            }
+          } else {
+            // the parent's bounds and the sibling the step leads to
+            const float s2 = bounds.size * 2.0f;
+            const float rcp_s2 = size_rcp<P2>(s2);
+            const V3f pmin{sub_fmod_size<P2>(bounds.min.x, s2, rcp_s2),
+                           sub_fmod_size<P2>(bounds.min.y, s2, rcp_s2),
+                           sub_fmod_size<P2>(bounds.min.z, s2, rcp_s2)};
+            next_target = step_octant_moved(pop_octant<P2>(bounds, pmin), moved, neg);
+            next_bounds = Cube{pmin, s2};
           }
-          st = dda_step(d, sig, &p, tb, scale);
-          next_target = step_octant(next_target, st);
-        }
-        if (guard) {
-          r.flags |= FLAG_ITERATION_GUARD;
-          break;
+        } else {
+          // the rest of ADVANCE
+          next_target = step_octant_moved(target, moved, neg);
+          if (++steps > t.max_steps) end = GUARD;
+          bp = V3f{rclamp(bp.x, lo, hi), rclamp(bp.y, lo, hi), rclamp(bp.z, lo, hi)};
+          V3f move = bitmap_move<P2>(
+              V3f{sx ? sig.x : 0.0f, sy ? sig.y : 0.0f, sz ? sig.z : 0.0f}, bounds.size,
+              rcp_size);
+          bool on = (next_target != OOB_OCTANT) & (end == RUNS);
+          while (on) {
+            tb = child_bounds_for(bounds, next_target);
+            bp = bp + move;
+            // stop at a reachable occupied child or a non-empty leaf brick;
+            // both words are requested together, whichever the test needs
+            const uint64_t there = lut[bitmap_index(bp, &r.flags) * 8u + dir_idx];
+            const uint32_t word = n.child[next_target];
+            const bool child = (kind == KIND_INTERNAL) &
+                               ((occ & octant_bitmap_mask(next_target)) != 0ull) &
+                               ((there & occ) != 0ull) & (word != INVALID_INDEX);
+            const bool brick =
+                (kind == KIND_LEAF) & (brick_form(meta, next_target) != FORM_EMPTY);
+            on = false;
+            if (!(child | brick)) {
+              if (++steps > t.max_steps) end = GUARD;
+              dda_step_axes(d, sig, &p, tb.min, tb.size, scale, &sx, &sy, &sz);
+              move = bitmap_move<P2>(
+                  V3f{sx ? sig.x : 0.0f, sy ? sig.y : 0.0f, sz ? sig.z : 0.0f}, bounds.size,
+                  rcp_size);
+              next_target = step_octant_moved(next_target, octant_of(sx, sy, sz), neg);
+              on = (next_target != OOB_OCTANT) & (end == RUNS);
+            }
+          }
         }
       }
+      // PUSH shifts the stack down (its oldest entry drops out once four are
+      // held), POP shifts it up, and a POP that empties it is followed by the
+      // restart's push of the root; ADVANCE leaves it
+      const uint32_t s0 = stk.s0, s1 = stk.s1, s2 = stk.s2, s3 = stk.s3;
+      stk.s0 = push ? tword : (pop ? (emptied ? 0u : s1) : s0);
+      stk.s1 = push ? s0 : (pop ? s2 : s1);
+      stk.s2 = push ? s1 : (pop ? s3 : s2);
+      stk.s3 = push ? s2 : s3;
+      stk.count = push ? (stk.count < 4u ? stk.count + 1u : 4u)
+                       : (pop ? (emptied ? 1u : stk.count - 1u) : stk.count);
+      if (LOD) mip_level += push ? -1.0f : (pop ? 1.0f : 0.0f);
+      bounds = next_bounds;
+      target = next_target;
+      // the next iteration would be one too many
+      if (end == RUNS && steps >= t.max_steps) end = GUARD;
     }
-    // PUSH shifts the stack down (its oldest entry drops out once four are
-    // held), POP shifts it up, and a POP that empties it is followed by the
-    // restart's push of the root; ADVANCE leaves it
-    const uint32_t s0 = stk.s0, s1 = stk.s1, s2 = stk.s2, s3 = stk.s3;
-    const bool emptied = pop && stk.count == 1u;
-    stk.s0 = push ? tword : (pop ? (emptied ? 0u : s1) : s0);
-    stk.s1 = push ? s0 : (pop ? s2 : s1);
-    stk.s2 = push ? s1 : (pop ? s3 : s2);
-    stk.s3 = push ? s2 : s3;
-    stk.count = push ? (stk.count < 4u ? stk.count + 1u : 4u)
-                     : (pop ? (emptied ? 1u : stk.count - 1u) : stk.count);
-    if (LOD) mip_level += push ? -1.0f : (pop ? 1.0f : 0.0f);
-    bounds = next_bounds;
-    target = next_target;
+  } while (end == RUNS);
+#if defined(__HIP_DEVICE_COMPILE__)
+  // (opaque here, so that the tests below are not carried through the loop)
+  asm volatile("" : "+v"(end));
+#endif
+  if (end == CRAWL) return crawl_out_of_root(t, p, d, steps, r.flags);
+  if (end == GUARD) r.flags |= FLAG_ITERATION_GUARD;
+  const bool mip = LOD && end == HIT_MIP;
+  if (end == HIT || mip) {
+    // the brick that was hit, from the state the hit left as it was
+    const NodeRec& n = (stk.s0 < ntop ? top : t.nodes)[stk.s0];
+    const uint32_t meta = n.meta;
+    const bool uniform = node_kind(meta) == KIND_UNIFORM_LEAF;
+    const bool whole = uniform || mip;
+    const uint32_t slot = uniform ? 0u : target & 7u;  // (unused by a MIP hit)
+    const Cube tb = child_bounds_for(bounds, target);
+    const Cube bb{V3f{whole ? bounds.min.x : tb.min.x, whole ? bounds.min.y : tb.min.y,
+                      whole ? bounds.min.z : tb.min.z},
+                  whole ? bounds.size : tb.size};
+    brick_hit<P2>(t, mip ? n.mip : brick_form(meta, slot), mip ? n.mip_word : n.child[slot], bb,
+                  cell, p, &r);
   }
-  if constexpr (LOD)
-    if (crawl) return crawl_out_of_root(t, p, d, steps, r.flags);
-  return miss_flags(r.flags);
-hit_found:
-  r.hit = 1;
   return r;
 }
 
