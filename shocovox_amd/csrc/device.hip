@@ -1,9 +1,9 @@
 // gfx950 kernels of the traversal path and device residency of a tree.
 //
 // cast_kernel: one ray per lane from a caller-provided ray array.
-// render_kernel: primary rays generated on the device; each 64-lane wave
-//   owns an 8x8 pixel tile so neighbouring lanes follow nearby paths through
-//   the tree and share node and brick cache lines.
+// frame_kernel: primary rays generated on the device; each wave owns a pixel
+//   tile so neighbouring lanes follow nearby paths through the tree and share
+//   node and brick cache lines. render_kernel: its selectable variants.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,31 +22,34 @@ namespace svo {
 
 namespace {
 
-// `order` (optional): lane i traverses ray order[i] (svo_cast's traversal
+// The plain kernels run one wave per workgroup (its slot is free as soon as it
+// ends; with four waves the fastest three wait for the slowest) and give a
+// wave 2^rays_log2 rays, its other lanes none (wave_rays_log2 says how many).
+
+// `order` (optional): the wave's k-th ray is order[k] (svo_cast's traversal
 // order for large ray sets, order.hip); each ray writes its own outputs.
-__global__ __launch_bounds__(256) void cast_kernel(TreeView t, const float* __restrict__ rays,
-                                                   uint32_t n, const uint32_t* __restrict__ order,
-                                                   HitPtrs out) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const uint32_t i = order ? order[k] : k;
+__global__ __launch_bounds__(64) void cast_kernel(TreeView t, const float* __restrict__ rays,
+                                                  uint32_t n, const uint32_t* __restrict__ order,
+                                                  uint32_t rays_log2, HitPtrs out) {
+  const uint64_t k = (static_cast<uint64_t>(blockIdx.x) << rays_log2) + threadIdx.x;
+  if ((threadIdx.x >> rays_log2) != 0u || k >= n) return;
+  const uint32_t i = order ? order[k] : static_cast<uint32_t>(k);
   const float* r = rays + 6ull * i;
   const V3f o{r[0], r[1], r[2]};
   const V3f d{r[3], r[4], r[5]};
-  const CastResult res = cast_ray_ww<true>(t, t.ray_lut, o, d, static_cast<const NodeRec*>(nullptr),
-                                           0u);
+  const CastResult res = cast_ray<true>(t, o, d);
   store_result(t, out, i, res, o);
 }
 
 // get_by_ray_at_lod for a ray array (MIP bricks probed per the viewing
 // distance when the tree's MIPs are enabled).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void cast_lod_kernel(TreeView t, const float* __restrict__ rays,
-                                                       uint32_t n, float viewing_distance,
-                                                       const uint32_t* __restrict__ order,
-                                                       HitPtrs out) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const uint32_t i = order ? order[k] : k;  // as in cast_kernel
+__global__ __launch_bounds__(64) void cast_lod_kernel(TreeView t, const float* __restrict__ rays,
+                                                      uint32_t n, float viewing_distance,
+                                                      const uint32_t* __restrict__ order,
+                                                      uint32_t rays_log2, HitPtrs out) {
+  const uint64_t k = (static_cast<uint64_t>(blockIdx.x) << rays_log2) + threadIdx.x;
+  if ((threadIdx.x >> rays_log2) != 0u || k >= n) return;
+  const uint32_t i = order ? order[k] : static_cast<uint32_t>(k);
   const float* r = rays + 6ull * i;
   const V3f o{r[0], r[1], r[2]};
   const V3f d{r[3], r[4], r[5]};
@@ -54,18 +57,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void c
   store_result(t, out, i, res, o);
 }
 
-// get_by_ray_at_lod for the primary rays of a viewport: four 64-lane waves
-// per workgroup, each over one 8x8 pixel tile.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void render_lod_kernel(TreeView t, Camera cam, uint32_t w,
-                                                         uint32_t h, float viewing_distance,
-                                                         HitPtrs out) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = threadIdx.x >> 6;
-  const uint32_t x = (blockIdx.x * 2u + (wave & 1u)) * 8u + (lane % 8u);
-  const uint32_t y = (blockIdx.y * 2u + (wave >> 1)) * 8u + (lane / 8u);
-  if (x >= w || y >= h) return;
-  const V3f d = camera_ray_dir(cam, x, y);
-  const CastResult res = cast_ray_lod<true>(t, t.ray_lut, cam.origin, d, viewing_distance);
+// A plain image kernel's tiles, one per workgroup in row order: 2^log_w x
+// 2^log_h pixels, one per lane. (The grid's second dimension only continues
+// the first, which holds fewer than 2^32 threads.)
+struct Tiles {
+  uint32_t log_w, log_h, per_row, count;
+};
+
+// The pixel of this lane; false when it has none.
+__device__ inline bool tile_pixel(const Tiles& tl, uint32_t w, uint32_t h, uint32_t* x,
+                                  uint32_t* y) {
+  const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
+  if (tile >= tl.count) return false;
+  const uint32_t ty = tile / tl.per_row, tx = tile - ty * tl.per_row;
+  *x = (tx << tl.log_w) + (threadIdx.x & ((1u << tl.log_w) - 1u));
+  *y = (ty << tl.log_h) + (threadIdx.x >> tl.log_w);
+  return (threadIdx.x >> (tl.log_w + tl.log_h)) == 0u && *x < w && *y < h;
+}
+
+// Primary rays of a viewport (svo_render's launch unless a variant is chosen).
+__global__ __launch_bounds__(64) void frame_kernel(TreeView t, Camera cam, uint32_t w, uint32_t h,
+                                                   Tiles tl, HitPtrs out) {
+  uint32_t x, y;
+  if (!tile_pixel(tl, w, h, &x, &y)) return;
+  const CastResult res = cast_ray<true>(t, cam.origin, camera_ray_dir(cam, x, y));
+  store_result(t, out, y * w + x, res, cam.origin);
+}
+
+// get_by_ray_at_lod for the primary rays of a viewport.
+__global__ __launch_bounds__(64) void frame_lod_kernel(TreeView t, Camera cam, uint32_t w,
+                                                       uint32_t h, float viewing_distance,
+                                                       Tiles tl, HitPtrs out) {
+  uint32_t x, y;
+  if (!tile_pixel(tl, w, h, &x, &y)) return;
+  const CastResult res =
+      cast_ray_lod<true>(t, t.ray_lut, cam.origin, camera_ray_dir(cam, x, y), viewing_distance);
   store_result(t, out, y * w + x, res, cam.origin);
 }
 
@@ -172,13 +198,11 @@ __device__ inline uint32_t unorm8(float v) {
 }
 
 template <int CONV>
-__global__ __launch_bounds__(256) void shade_kernel(TreeView t, ShadeParams sp, uint32_t w,
-                                                    uint32_t h, uint32_t* __restrict__ out) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = threadIdx.x >> 6;
-  const uint32_t x = (blockIdx.x * 2u + (wave & 1u)) * 8u + (lane & 7u);
-  const uint32_t row = (blockIdx.y * 2u + (wave >> 1)) * 8u + (lane >> 3);
-  if (x >= w || row >= h) return;
+__global__ __launch_bounds__(64) void shade_kernel(TreeView t, ShadeParams sp, uint32_t w,
+                                                   uint32_t h, Tiles tl,
+                                                   uint32_t* __restrict__ out) {
+  uint32_t x, row;
+  if (!tile_pixel(tl, w, h, &x, &row)) return;
   V3f o, d;
   if (CONV == 0) {
     const uint32_t y = h - 1u - row;
@@ -194,8 +218,7 @@ __global__ __launch_bounds__(256) void shade_kernel(TreeView t, ShadeParams sp, 
     o = glass;
     d = normalized(glass - sp.origin);
   }
-  const CastResult r =
-      cast_ray_ww<true>(t, t.ray_lut, o, d, static_cast<const NodeRec*>(nullptr), 0u);
+  const CastResult r = cast_ray<true>(t, o, d);
   uint32_t rgba;
   if (r.hit) {
     const uint32_t ci = pix_color_index(r.pix);
@@ -263,14 +286,47 @@ const RenderVariant kRenderVariants[] = {
     // 1080p primary rays (lanes drift apart and lose the shared node lines);
     // kept as a variant for divergent workloads
     {"r1-t4-f16", render_refill_kernel<1, 4, 16>, 8, 8, 4},
+    // frame_kernel, its tiles chosen by the image's size (wave_rays_log2)
+    {"auto", nullptr, 0, 0},
 };
 constexpr int kRenderVariantCount = sizeof(kRenderVariants) / sizeof(kRenderVariants[0]);
-int initial_render_variant() {
-  for (int i = 0; i < kRenderVariantCount; ++i)
-    if (std::strcmp(kRenderVariants[i].name, "w6-slut-8x8-ww") == 0) return i;
-  return 0;
+constexpr int kAutoVariant = kRenderVariantCount - 1;
+int g_render_variant = kAutoVariant;
+
+// log2 of the rays a wave of a plain launch takes: 64 once that makes 2048
+// waves (two per SIMD), fewer, down to 4, for smaller launches. Such a launch
+// lasts as long as its slowest wave, and a wave runs the paths of all its
+// lanes, so a chip with idle SIMDs answers sooner with its rays spread over
+// more waves; beyond about two waves per SIMD the extra instructions cost
+// more. Microseconds with 64 / 32 / 16 / 8 / 4 / 2 rays a wave: 1,009 rays
+// 46 / 39 / 33 / 29 / 28 / 28; 60,000 rays 116 / 96 / 110 / 113 / 123 / 142;
+// a 256x256 frame 75 / 70 / 71 / 71 / 72 / 90; 300,007 rays 152 / 177 / 216.
+uint32_t wave_rays_log2(uint64_t rays) {
+  uint32_t k = 2;
+  while (k < 6 && rays > (uint64_t(2048) << k)) ++k;
+  return k;
 }
-int g_render_variant = initial_render_variant();
+
+// Workgroups of a plain launch over n rays.
+dim3 wave_grid(uint32_t n, uint32_t rays_log2) {
+  return dim3(static_cast<uint32_t>((static_cast<uint64_t>(n) + (1u << rays_log2) - 1u) >>
+                                    rays_log2));
+}
+
+Tiles tiles_for(uint32_t w, uint32_t h) {
+  const uint32_t k = wave_rays_log2(static_cast<uint64_t>(w) * h);
+  Tiles tl;
+  tl.log_w = (k + 1u) / 2u;
+  tl.log_h = k / 2u;
+  tl.per_row = (w >> tl.log_w) + ((w & ((1u << tl.log_w) - 1u)) != 0u);
+  tl.count = tl.per_row * ((h >> tl.log_h) + ((h & ((1u << tl.log_h) - 1u)) != 0u));
+  return tl;
+}
+// Grid of a plain image launch (w, h > 0, fewer than 2^32 pixels).
+dim3 tile_grid(const Tiles& tl) {
+  constexpr uint32_t kRow = 1u << 25;  // workgroups of 64: 2^31 threads
+  return tl.count <= kRow ? dim3(tl.count) : dim3(kRow, (tl.count + kRow - 1u) / kRow);
+}
 
 // Scatter of patched records: src[i] -> dst[idx[i]] (16-byte quarters per lane)
 __global__ __launch_bounds__(256) void scatter_records_kernel(NodeRec* __restrict__ dst,
@@ -441,7 +497,9 @@ int render_variant_scratch(int i, uint32_t* bytes, std::string* err) {
   }
   hipFuncAttributes a{};
   const hipError_t e =
-      hipFuncGetAttributes(&a, reinterpret_cast<const void*>(kRenderVariants[i].fn));
+      hipFuncGetAttributes(&a, i == kAutoVariant
+                                   ? reinterpret_cast<const void*>(frame_kernel)
+                                   : reinterpret_cast<const void*>(kRenderVariants[i].fn));
   if (e != hipSuccess) return hip_fail(e, "hipFuncGetAttributes", err);
   *bytes = static_cast<uint32_t>(a.localSizeBytes);
   return SVO_OK;
@@ -970,11 +1028,8 @@ int device_cast(const DeviceTree& t, const float* rays, uint32_t n, const svo_hi
     const int st = order_rays(rays, n, t.view.size, &order, s, err);
     if (st != SVO_OK && st != SVO_OUT_OF_DEVICE_MEMORY) return st;
   }
-  // n < 2^32, so the grid (at most 2^24 workgroups) is computed without
-  // wrapping in 64 bits
-  const uint32_t block = 256;
-  const uint32_t grid = static_cast<uint32_t>((static_cast<uint64_t>(n) + block - 1) / block);
-  hipLaunchKernelGGL(cast_kernel, dim3(grid), dim3(block), 0, s, t.view, rays, n, order,
+  const uint32_t k = wave_rays_log2(n);
+  hipLaunchKernelGGL(cast_kernel, wave_grid(n, k), dim3(64), 0, s, t.view, rays, n, order, k,
                      to_ptrs(out));
   hipError_t e = hipGetLastError();
   if (order) (void)hipFreeAsync(order, s);
@@ -1005,9 +1060,9 @@ int device_cast_lod(const DeviceTree& t, const float* rays, uint32_t n, float vi
     const int st = order_rays(rays, n, t.view.size, &order, s, err);
     if (st != SVO_OK && st != SVO_OUT_OF_DEVICE_MEMORY) return st;
   }
-  const uint32_t grid = static_cast<uint32_t>((static_cast<uint64_t>(n) + 255u) / 256u);
-  hipLaunchKernelGGL(cast_lod_kernel, dim3(grid), dim3(256), 0, s, t.view, rays, n,
-                     viewing_distance, order, to_ptrs(out));
+  const uint32_t k = wave_rays_log2(n);
+  hipLaunchKernelGGL(cast_lod_kernel, wave_grid(n, k), dim3(64), 0, s, t.view, rays, n,
+                     viewing_distance, order, k, to_ptrs(out));
   hipError_t e = hipGetLastError();
   if (order) (void)hipFreeAsync(order, s);
   if (e != hipSuccess) return hip_fail(e, "cast_lod_kernel launch", err);
@@ -1022,11 +1077,11 @@ int device_render_lod(const DeviceTree& t, const Camera& cam, uint32_t w, uint32
   if (!image_fits(w, h, err)) return SVO_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
-  const dim3 grid((w + 15u) / 16u, (h + 15u) / 16u);
-  hipLaunchKernelGGL(render_lod_kernel, grid, dim3(256), 0, s, t.view, cam, w, h,
-                     viewing_distance, to_ptrs(out));
+  const Tiles tl = tiles_for(w, h);
+  hipLaunchKernelGGL(frame_lod_kernel, tile_grid(tl), dim3(64), 0, s, t.view, cam, w, h,
+                     viewing_distance, tl, to_ptrs(out));
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return hip_fail(e, "render_lod_kernel launch", err);
+  if (e != hipSuccess) return hip_fail(e, "frame_lod_kernel launch", err);
   timer.done();
   return SVO_OK;
 }
@@ -1037,6 +1092,15 @@ int device_render(const DeviceTree& t, const Camera& cam, uint32_t w, uint32_t h
   if (!image_fits(w, h, err)) return SVO_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
+  if (g_render_variant == kAutoVariant) {
+    const Tiles tl = tiles_for(w, h);
+    hipLaunchKernelGGL(frame_kernel, tile_grid(tl), dim3(64), 0, s, t.view, cam, w, h, tl,
+                       to_ptrs(out));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "frame_kernel launch", err);
+    timer.done();
+    return SVO_OK;
+  }
   const RenderVariant& v = kRenderVariants[g_render_variant];
   const uint32_t gx = v.single_wave_groups ? 1u : 2u;
   dim3 grid((w + gx * v.tile_w - 1) / (gx * v.tile_w), (h + gx * v.tile_h - 1) / (gx * v.tile_h));
@@ -1092,11 +1156,13 @@ int device_render_rgba8(const DeviceTree& t, V3f origin, V3f dir, float glass_w,
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
-  const dim3 grid((w + 15) / 16, (h + 15) / 16);
+  const Tiles tl = tiles_for(w, h);
   if (convention == 0)
-    hipLaunchKernelGGL(shade_kernel<0>, grid, dim3(256), 0, s, t.view, sp, w, h, out);
+    hipLaunchKernelGGL(shade_kernel<0>, tile_grid(tl), dim3(64), 0, s, t.view, sp, w, h, tl,
+                       out);
   else
-    hipLaunchKernelGGL(shade_kernel<1>, grid, dim3(256), 0, s, t.view, sp, w, h, out);
+    hipLaunchKernelGGL(shade_kernel<1>, tile_grid(tl), dim3(64), 0, s, t.view, sp, w, h, tl,
+                       out);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "shade_kernel launch", err);
   timer.done();
