@@ -1,27 +1,31 @@
-// Batched mode: every tile of every job in one persistent launch.
+// Batched mode: every tile of every job in one launch.
 //
 // A job is a viewport render or a ray-array cast on one resident tree. Its
 // rays are cut into 64-ray tiles (8x8 pixels for renders), numbered
-// contiguously across jobs. The tile space is split into 8 contiguous
-// chunks, one per XCD (workgroups are dispatched to the 8 XCDs round-robin),
-// so neighbouring tiles - which touch the same nodes and bricks - are served
-// by one XCD's L2. Each wave takes the next tiles of its XCD's chunk from a
-// device counter and, once that chunk is exhausted, steals from the other
-// chunks; every wave leaves when all chunks are empty.
+// contiguously across jobs. The default kernel ("auto", batch_tile_kernel)
+// has one one-wave workgroup per tile, which the hardware hands out in order.
+// The persistent variants split the tile space into 8 contiguous chunks, one
+// per XCD (workgroups are dispatched to the 8 XCDs round-robin); each wave
+// takes the next tiles of its XCD's chunk from a device counter and, once that
+// chunk is exhausted, steals from the other chunks; every wave leaves when all
+// chunks are empty. Their counters cost a device-wide atomic round trip per
+// tile and, at the end, one per wave and chunk (4,096 waves x 8): 8 1080p
+// frames 0.81 ms with the best of them and 0.92 with the former default
+// against 0.74 per tile, one 320x240 frame 0.20 against 0.14 ms.
 //
-// Kernel variants: "classic" takes one tile per grab and runs it as one ray
+// Persistent variants: "classic" takes one tile per grab and runs it as one ray
 // per lane (with an occupancy hint of 1 or 5 waves per SIMD), "ww" likewise
 // with the while-while form of the traversal (cast_ray_ww); the refill
 // variants take TPW tiles per grab and run them with lane refill
 // (refill.hpp), one job segment at a time.
 //
-// The per-run sequence - job table upload from pinned memory (only the bytes
-// the run uses), counter reset (a fill kernel, not a memset), persistent
-// kernel - is a hipGraph built once per context; each run sets the copy's
-// source and size and replays it. Two pinned stagings alternate, so the host
+// A run writes its job table to the device (by kernel arguments when it is
+// small, else from pinned memory) and launches the kernel; the persistent
+// variants replay a hipGraph built once per context (table copy, counter
+// reset by a fill kernel, kernel). Two pinned stagings alternate, so the host
 // fills the next run's table while the previous run executes; a run waits on
 // its stream for the previous run (which may have been issued on another
-// stream) before its copy overwrites the device table.
+// stream) before it overwrites the device table.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -54,7 +58,8 @@ struct alignas(16) BatchJob {
   uint32_t first_tile;  // render: first image tile of the job
   uint32_t tile_major;  // 1: outputs stored tile after tile from out[0]
   float viewing_distance;  // > 0: get_by_ray_at_lod with this distance
-  uint32_t pad[2];
+  uint32_t tiles_x_rcp;    // floor((2^32 - 1) / tiles_x), for tile_row
+  uint32_t pad;
   Camera cam;
   const float* rays;
   // cast jobs: the traversal order of the rays (lane k of the job's tiles
@@ -63,12 +68,17 @@ struct alignas(16) BatchJob {
   HitPtrs out;
 };
 
-// Table of one run: [header][jobs x njobs][trees x ntrees]
+// Table of one run: [header][jobs x njobs][index x njobs][trees x ntrees]
 struct alignas(16) BatchHeader {
   uint32_t njobs;
   uint32_t total_tiles;
   uint32_t chunk_tiles;   // tiles per XCD chunk (the last chunk may be shorter)
   uint32_t trees_offset;  // byte offset of the tree table
+};
+// What the per-tile kernel finds a tile's job and tree by.
+struct BatchIndex {
+  uint32_t tile_begin;
+  uint32_t tree;
 };
 constexpr size_t kJobsOffset = 256;
 
@@ -90,6 +100,16 @@ __device__ inline uint32_t find_job(const BatchJob* jobs, uint32_t njobs, uint32
   return lo;
 }
 
+// Image row (of tiles) of a render job's tile; its column in *col. The
+// estimate is the quotient or one less (tiles are numbered below 2^26).
+__device__ inline uint32_t tile_row(const BatchJob& job, uint32_t image_tile, uint32_t* col) {
+  const uint32_t q = __umulhi(image_tile, job.tiles_x_rcp);
+  const uint32_t r = image_tile - q * job.tiles_x;
+  const bool more = r >= job.tiles_x;
+  *col = more ? r - job.tiles_x : r;
+  return more ? q + 1u : q;
+}
+
 __global__ __launch_bounds__(64) void reset_counters_kernel(Counter* counters) {
   if (threadIdx.x < kChunks) counters[threadIdx.x].next = 0u;
 }
@@ -104,10 +124,105 @@ __device__ inline const TreeView* trees_of(const char* table) {
   return reinterpret_cast<const TreeView*>(table + header_of(table)->trees_offset);
 }
 
+// Lane `lane` of a job's tile `local`: its ray's traversal and result. Render
+// jobs are cut into TW x TH pixel tiles (64 pixels, one per lane).
+template <bool WW, bool LOD, int TW, int TH>
+__device__ __attribute__((always_inline)) inline void cast_tile(const BatchJob& job,
+                                                                const TreeView& view,
+                                                                uint32_t local, uint32_t lane,
+                                                                const NodeRec* cache,
+                                                                uint32_t ntop) {
+  const TreeView tv = held_view(view);
+  // one inlined traversal serves both job kinds
+  V3f o, d;
+  uint32_t idx;
+  bool valid;
+  if (job.kind == 0) {
+    uint32_t col;
+    const uint32_t row = tile_row(job, local + job.first_tile, &col);
+    const uint32_t x = col * TW + (lane % TW);
+    const uint32_t y = row * TH + (lane / TW);
+    valid = x < job.width && y < job.height;
+    o = job.cam.origin;
+    d = valid ? camera_ray_dir(job.cam, x, y) : V3f{0.0f, 0.0f, 0.0f};
+    idx = job.tile_major ? local * 64u + lane : y * job.width + x;
+  } else {
+    idx = local * 64u + lane;
+    valid = idx < job.width;
+    if (valid && job.order) idx = as_global(job.order)[idx];
+    const float* rr = as_global(job.rays) + 6ull * (valid ? idx : 0u);
+    o = V3f{rr[0], rr[1], rr[2]};
+    d = V3f{rr[3], rr[4], rr[5]};
+  }
+  if (!valid) return;
+  CastResult r;
+  if constexpr (LOD) {
+    if (job.viewing_distance > 0.0f)
+      r = cast_ray_lod<true>(tv, tv.ray_lut, o, d, job.viewing_distance);
+    else
+      r = cast_ray<true>(tv, o, d);
+  } else if constexpr (WW) {
+    r = cast_ray_ww<true>(tv, tv.ray_lut, o, d, cache, ntop);
+  } else {
+    r = cast_ray<true>(tv, tv.ray_lut, o, d, cache, ntop);
+  }
+  // The origin and the output index are formed again for the store rather
+  // than carried through the traversal (four registers fewer there): the
+  // empty asm hides that `local` is unchanged, so the compiler recomputes
+  // them (a render's origin is the job's camera, a cast's is read again from
+  // its ray).
+  uint32_t again = local;
+  asm volatile("" : "+s"(again));
+  if (job.kind == 0) {
+    uint32_t col;
+    const uint32_t row = tile_row(job, again + job.first_tile, &col);
+    const uint32_t x = col * TW + (lane % TW);
+    const uint32_t y = row * TH + (lane / TW);
+    o = job.cam.origin;
+    idx = job.tile_major ? again * 64u + lane : y * job.width + x;
+  } else {
+    idx = again * 64u + lane;
+    if (job.order) idx = as_global(job.order)[idx];
+    const float* rr = as_global(job.rays) + 6ull * idx;
+    o = V3f{rr[0], rr[1], rr[2]};
+  }
+  store_result(tv, held_ptrs(job.out), idx, r, o);
+}
+
+// One wave per workgroup over one tile, or over 2^rays_log2 of its rays: the
+// hardware hands out the tiles, in order, as slots fall free. The wave's lanes
+// compare the tile with 64 jobs' first tiles at once (in the block of 64 that
+// a binary search leaves), and the tree's index comes with them, so that the
+// job and its tree are read side by side: a wave starts three memory round
+// trips after its launch.
+template <int MIN_WAVES, bool LOD>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
+void batch_tile_kernel(const char* __restrict__ table, uint32_t njobs, uint32_t index_offset,
+                       uint32_t trees_offset, uint32_t rays_log2) {
+  const uint32_t tile = blockIdx.x >> (6u - rays_log2);
+  const BatchIndex* index = reinterpret_cast<const BatchIndex*>(table + index_offset);
+  uint32_t block = 0, blocks = (njobs + 63u) >> 6;
+  while (blocks > 1u) {
+    const uint32_t half = blocks >> 1;
+    const bool upper = index[(block + half) << 6].tile_begin <= tile;
+    block = upper ? block + half : block;
+    blocks = upper ? blocks - half : half;
+  }
+  const uint32_t slot = (block << 6) + threadIdx.x;
+  const BatchIndex mine = index[min(slot, njobs - 1u)];
+  const uint64_t begun = __ballot(slot < njobs && mine.tile_begin <= tile);
+  const uint32_t last = 63u - static_cast<uint32_t>(__builtin_clzll(begun));
+  const uint32_t tree = __builtin_amdgcn_readlane(mine.tree, last);
+  const BatchJob& job = jobs_of(table)[(block << 6) + last];
+  const TreeView& tv = reinterpret_cast<const TreeView*>(table + trees_offset)[tree];
+  if ((threadIdx.x >> rays_log2) != 0u) return;
+  const uint32_t lane = ((blockIdx.x << rays_log2) & 63u) + threadIdx.x;
+  cast_tile<false, LOD, 8, 8>(job, tv, tile - job.tile_begin, lane, nullptr, 0u);
+}
+
 // LOD compiles in get_by_ray_at_lod for jobs with a viewing distance; a
 // context launches that form only for runs that hold such jobs, so the plain
 // form keeps its smaller register allocation.
-// Render jobs are cut into TW x TH pixel tiles (64 pixels, one per lane).
 // NODES > 0 stages the first NODES node records of a tree (the top levels of
 // the breadth-first numbering) in LDS, where the traversal reads them:
 // without SHARED each wave keeps the records of the tree of its current job
@@ -175,59 +290,7 @@ void batch_kernel(const char* __restrict__ table, Counter* __restrict__ counters
         }
       }
       const uint32_t ntop = NODES > 0 && job.tree == cached_tree ? ncached : 0u;
-      // the lane's ray; one inlined traversal serves both job kinds
-      V3f o, d;
-      uint32_t idx;
-      bool valid;
-      if (job.kind == 0) {
-        const uint32_t image_tile = local + job.first_tile;
-        const uint32_t x = (image_tile % job.tiles_x) * TW + (lane % TW);
-        const uint32_t y = (image_tile / job.tiles_x) * TH + (lane / TW);
-        valid = x < job.width && y < job.height;
-        o = job.cam.origin;
-        d = valid ? camera_ray_dir(job.cam, x, y) : V3f{0.0f, 0.0f, 0.0f};
-        idx = job.tile_major ? local * 64u + lane : y * job.width + x;
-      } else {
-        idx = local * 64u + lane;
-        valid = idx < job.width;
-        if (valid && job.order) idx = job.order[idx];
-        const float* rr = job.rays + 6ull * (valid ? idx : 0u);
-        o = V3f{rr[0], rr[1], rr[2]};
-        d = V3f{rr[3], rr[4], rr[5]};
-      }
-      if (valid) {
-        CastResult r;
-        if constexpr (LOD) {
-          if (job.viewing_distance > 0.0f)
-            r = cast_ray_lod<true>(tv, tv.ray_lut, o, d, job.viewing_distance);
-          else
-            r = cast_ray<true>(tv, o, d);
-        } else if constexpr (WW) {
-          r = cast_ray_ww<true>(tv, tv.ray_lut, o, d, static_cast<const NodeRec*>(cache), ntop);
-        } else {
-          r = cast_ray<true>(tv, tv.ray_lut, o, d, static_cast<const NodeRec*>(cache), ntop);
-        }
-        // The origin and the output index are formed again for the store
-        // rather than carried through the traversal (four registers fewer
-        // there): the empty asm hides that `local` is unchanged, so the
-        // compiler recomputes them (a render's origin is the job's camera,
-        // a cast's is read again from its ray).
-        uint32_t again = local;
-        asm volatile("" : "+s"(again));
-        if (job.kind == 0) {
-          const uint32_t image_tile = again + job.first_tile;
-          const uint32_t x = (image_tile % job.tiles_x) * TW + (lane % TW);
-          const uint32_t y = (image_tile / job.tiles_x) * TH + (lane / TW);
-          o = job.cam.origin;
-          idx = job.tile_major ? again * 64u + lane : y * job.width + x;
-        } else {
-          idx = again * 64u + lane;
-          if (job.order) idx = job.order[idx];
-          const float* rr = job.rays + 6ull * idx;
-          o = V3f{rr[0], rr[1], rr[2]};
-        }
-        store_result(tv, job.out, idx, r, o);
-      }
+      cast_tile<WW, LOD, TW, TH>(job, tv, local, lane, cache, ntop);
     }
   }
 }
@@ -285,6 +348,7 @@ struct BatchVariant {
   uint32_t groups_per_cu;  // 256-lane workgroups per CU in the persistent grid
   uint32_t tile_w, tile_h; // pixel tile of render jobs
   bool orders_casts = true;  // its kernel takes a cast job's traversal order
+  bool per_tile = false;     // a workgroup per tile (batch_tile_kernel), not a persistent grid
 };
 
 // runs that hold get_by_ray_at_lod jobs use the LOD form of the variant's
@@ -313,17 +377,54 @@ const BatchVariant kBatchVariants[] = {
     // six waves per SIMD (at most 80 VGPRs)
     {"classic-w6-g6", batch_kernel<6>, kLod8x8, 6, 8, 8},
     {"classic-w6-g6-n73", batch_kernel<6, false, false, 8, 8, 73>, kLod8x8, 6, 8, 8},
+    {"auto", nullptr, nullptr, 0, 8, 8, true, true},
 };
 constexpr int kBatchVariantCount = sizeof(kBatchVariants) / sizeof(kBatchVariants[0]);
-int g_batch_variant = 0;
+int g_batch_variant = kBatchVariantCount - 1;
+
+// One upload kernel carries up to 3 KiB of the table in its arguments
+// (kernel arguments are limited to 4 KiB).
+constexpr uint32_t kUploadWords = 768;
+struct UploadChunk {
+  uint32_t offset_words;
+  uint32_t count;
+  uint32_t words[kUploadWords];
+};
+
+__global__ __launch_bounds__(256) void upload_table_kernel(uint32_t* __restrict__ dst,
+                                                           const UploadChunk c) {
+  for (uint32_t i = threadIdx.x; i < c.count; i += 256u) dst[c.offset_words + i] = c.words[i];
+}
+
+// Writes `bytes` of a table (a multiple of 4) to the device by upload kernels.
+void upload_table(void* dst, const char* src, size_t bytes, hipStream_t s) {
+  const uint32_t words = static_cast<uint32_t>((bytes + 3) / 4);
+  for (uint32_t w0 = 0; w0 < words; w0 += kUploadWords) {
+    UploadChunk c;
+    c.offset_words = w0;
+    c.count = std::min(kUploadWords, words - w0);
+    std::memcpy(c.words, src + static_cast<size_t>(w0) * 4, static_cast<size_t>(c.count) * 4);
+    hipLaunchKernelGGL(upload_table_kernel, dim3(1), dim3(256), 0, s,
+                       static_cast<uint32_t*>(dst), c);
+  }
+}
+
+// Tables up to this size go by upload kernels (four of them), larger ones by a
+// copy; the two measured alike at 1 to 24 jobs, and the kernels need no
+// staging.
+constexpr size_t kUploadBytes = 12 << 10;
+
 
 int hip_fail(hipError_t e, const char* what, std::string* err) {
   *err = std::string(what) + ": " + hipGetErrorString(e);
   return e == hipErrorOutOfMemory ? SVO_OUT_OF_DEVICE_MEMORY : SVO_HIP_ERROR;
 }
 
-constexpr size_t trees_offset_for(uint32_t njobs) {
+constexpr size_t index_offset_for(uint32_t njobs) {
   return (kJobsOffset + njobs * sizeof(BatchJob) + 63) & ~size_t(63);
+}
+constexpr size_t trees_offset_for(uint32_t njobs) {
+  return (index_offset_for(njobs) + njobs * sizeof(BatchIndex) + 63) & ~size_t(63);
 }
 
 // Table entry of job `in` on tree slot `ti`, its tiles numbered from `*tiles`
@@ -341,6 +442,7 @@ int fill_job(BatchJob& j, const BatchJobIn& in, uint32_t ti, uint32_t tw, uint32
       return SVO_INVALID_ARGUMENT;
     }
     j.tiles_x = (in.width + tw - 1) / tw;
+    j.tiles_x_rcp = j.tiles_x ? 0xFFFFFFFFu / j.tiles_x : 0u;
     const uint64_t image_tiles = static_cast<uint64_t>(j.tiles_x) * ((in.height + th - 1) / th);
     const uint64_t limit = in.tile_limit ? in.tile_limit : image_tiles - std::min<uint64_t>(
                                                                 in.first_tile, image_tiles);
@@ -377,12 +479,33 @@ int fill_job(BatchJob& j, const BatchJobIn& in, uint32_t ti, uint32_t tw, uint32
   return SVO_OK;
 }
 
+// Header and index of a table whose jobs are filled in.
 void fill_header(char* base, uint32_t n, uint64_t tiles, size_t trees_offset) {
+  const BatchJob* jobs = reinterpret_cast<const BatchJob*>(base + kJobsOffset);
+  BatchIndex* index = reinterpret_cast<BatchIndex*>(base + index_offset_for(n));
+  for (uint32_t i = 0; i < n; ++i) index[i] = BatchIndex{jobs[i].tile_begin, jobs[i].tree};
   BatchHeader* hdr = reinterpret_cast<BatchHeader*>(base);
   hdr->njobs = n;
   hdr->total_tiles = static_cast<uint32_t>(tiles);
   hdr->chunk_tiles = static_cast<uint32_t>((tiles + kChunks - 1) / kChunks);
   hdr->trees_offset = static_cast<uint32_t>(trees_offset);
+}
+
+// Launches the per-tile kernel over the tiles (fewer than 2^26) of a table of
+// n jobs.
+hipError_t launch_tiles(const char* table, uint32_t n, uint64_t tiles, bool lod, hipStream_t s) {
+  if (tiles == 0) return hipSuccess;
+  const uint32_t k = wave_rays_log2(tiles * 64);
+  const dim3 grid(static_cast<uint32_t>(tiles << (6u - k)));
+  const uint32_t index = static_cast<uint32_t>(index_offset_for(n));
+  const uint32_t trees = static_cast<uint32_t>(trees_offset_for(n));
+  if (lod)
+    hipLaunchKernelGGL((batch_tile_kernel<6, true>), grid, dim3(64), 0, s, table, n, index, trees,
+                       k);
+  else
+    hipLaunchKernelGGL((batch_tile_kernel<8, false>), grid, dim3(64), 0, s, table, n, index,
+                       trees, k);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -465,7 +588,9 @@ int batch_variant_scratch(int i, uint32_t* bytes, std::string* err) {
   }
   hipFuncAttributes a{};
   const hipError_t e =
-      hipFuncGetAttributes(&a, reinterpret_cast<const void*>(kBatchVariants[i].fn));
+      hipFuncGetAttributes(&a, kBatchVariants[i].per_tile
+                                   ? reinterpret_cast<const void*>(batch_tile_kernel<8, false>)
+                                   : reinterpret_cast<const void*>(kBatchVariants[i].fn));
   if (e != hipSuccess) {
     *err = std::string("hipFuncGetAttributes: ") + hipGetErrorString(e);
     return SVO_HIP_ERROR;
@@ -526,11 +651,13 @@ int batch_create_variant(uint32_t max_jobs, int variant, BatchContext** out, std
   std::memset(b->host[1], 0, b->table_bytes);
   // groups_per_cu 256-lane workgroups per CU: that many waves on every SIMD
   b->grid = static_cast<uint32_t>(std::max(cus, 1)) * kBatchVariants[b->variant].groups_per_cu;
-  const int st = build_graph(b, kBatchVariants[b->variant].fn, &b->graph, &b->copy_node,
-                             &b->exec, err);
-  if (st != SVO_OK) {
-    batch_destroy(b);
-    return st;
+  if (!kBatchVariants[b->variant].per_tile) {
+    const int st = build_graph(b, kBatchVariants[b->variant].fn, &b->graph, &b->copy_node,
+                               &b->exec, err);
+    if (st != SVO_OK) {
+      batch_destroy(b);
+      return st;
+    }
   }
   *out = b;
   return SVO_OK;
@@ -618,7 +745,8 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
   fill_header(base, n, tiles, trees_offset);
   b->last_tiles = tiles;
   const size_t used = trees_offset + tree_index.size() * sizeof(TreeView);
-  if (any_lod && !b->exec_lod) {
+  const bool per_tile = kBatchVariants[b->variant].per_tile;
+  if (any_lod && !per_tile && !b->exec_lod) {
     const int st = build_graph(b, kBatchVariants[b->variant].lod_fn, &b->graph_lod,
                                &b->copy_node_lod, &b->exec_lod, err);
     if (st != SVO_OK) {
@@ -626,11 +754,21 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
       return st;
     }
   }
-  hipGraphExec_t exec = any_lod ? b->exec_lod : b->exec;
-  hipError_t e = hipGraphExecMemcpyNodeSetParams1D(
-      exec, any_lod ? b->copy_node_lod : b->copy_node, b->dev, base, used, hipMemcpyHostToDevice);
-  if (e == hipSuccess && b->pending[slot ^ 1u]) e = hipStreamWaitEvent(s, b->done[slot ^ 1u], 0);
-  if (e == hipSuccess) e = hipGraphLaunch(exec, s);
+  hipError_t e = hipSuccess;
+  if (b->pending[slot ^ 1u]) e = hipStreamWaitEvent(s, b->done[slot ^ 1u], 0);
+  if (per_tile) {
+    if (e == hipSuccess && used <= kUploadBytes)
+      upload_table(b->dev, base, used, s);
+    else if (e == hipSuccess)
+      e = hipMemcpyAsync(b->dev, base, used, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = launch_tiles(static_cast<const char*>(b->dev), n, tiles, any_lod, s);
+  } else {
+    hipGraphExec_t exec = any_lod ? b->exec_lod : b->exec;
+    if (e == hipSuccess)
+      e = hipGraphExecMemcpyNodeSetParams1D(exec, any_lod ? b->copy_node_lod : b->copy_node,
+                                            b->dev, base, used, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipGraphLaunch(exec, s);
+  }
   for (uint32_t* p : orders) (void)hipFreeAsync(p, s);
   if (e != hipSuccess) return hip_fail(e, "batch launch", err);
   e = hipEventRecord(b->done[slot], s);
@@ -663,20 +801,6 @@ constexpr size_t kScratchBytes = kStaticCountersOffset + kChunks * sizeof(Counte
 static __device__ __align__(256) char scratch[kScratchBytes];
 
 namespace {
-
-// One upload kernel carries up to 3 KiB of the table in its arguments
-// (kernel arguments are limited to 4 KiB).
-constexpr uint32_t kUploadWords = 768;
-struct UploadChunk {
-  uint32_t offset_words;
-  uint32_t count;
-  uint32_t words[kUploadWords];
-};
-
-__global__ __launch_bounds__(256) void upload_table_kernel(uint32_t* __restrict__ dst,
-                                                           const UploadChunk c) {
-  for (uint32_t i = threadIdx.x; i < c.count; i += 256u) dst[c.offset_words + i] = c.words[i];
-}
 
 constexpr int kStaticMaxDevices = 64;
 struct StaticDevice {
@@ -772,22 +896,18 @@ int run_static(const svo_job* jobs, uint32_t n, void* stream, std::string* err) 
   fill_header(base, n, tiles, trees_offset);
   const size_t used = trees_offset + ntrees * sizeof(TreeView);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  uint32_t* dst = reinterpret_cast<uint32_t*>(sd->scratch);
-  const uint32_t words = static_cast<uint32_t>((used + 3) / 4);
-  for (uint32_t w0 = 0; w0 < words; w0 += kUploadWords) {
-    UploadChunk c;
-    c.offset_words = w0;
-    c.count = std::min(kUploadWords, words - w0);
-    std::memcpy(c.words, base + static_cast<size_t>(w0) * 4, static_cast<size_t>(c.count) * 4);
-    hipLaunchKernelGGL(upload_table_kernel, dim3(1), dim3(256), 0, s, dst, c);
-  }
-  Counter* counters = reinterpret_cast<Counter*>(sd->scratch + kStaticCountersOffset);
-  hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, s, counters);
+  upload_table(sd->scratch, base, used, s);
   const BatchVariant& v = kBatchVariants[g_batch_variant];
-  const BatchFn fn = any_lod ? v.lod_fn : v.fn;
-  const uint32_t grid = sd->cus * v.groups_per_cu;
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, s, static_cast<const char*>(sd->scratch),
-                     counters);
+  if (v.per_tile) {
+    (void)launch_tiles(sd->scratch, n, tiles, any_lod, s);
+  } else {
+    Counter* counters = reinterpret_cast<Counter*>(sd->scratch + kStaticCountersOffset);
+    hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, s, counters);
+    const BatchFn fn = any_lod ? v.lod_fn : v.fn;
+    const uint32_t grid = sd->cus * v.groups_per_cu;
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, s, static_cast<const char*>(sd->scratch),
+                       counters);
+  }
   e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "svo_batch_run_static launch", err);
   return SVO_OK;

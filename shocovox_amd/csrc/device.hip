@@ -293,20 +293,6 @@ constexpr int kRenderVariantCount = sizeof(kRenderVariants) / sizeof(kRenderVari
 constexpr int kAutoVariant = kRenderVariantCount - 1;
 int g_render_variant = kAutoVariant;
 
-// log2 of the rays a wave of a plain launch takes: 64 once that makes 2048
-// waves (two per SIMD), fewer, down to 4, for smaller launches. Such a launch
-// lasts as long as its slowest wave, and a wave runs the paths of all its
-// lanes, so a chip with idle SIMDs answers sooner with its rays spread over
-// more waves; beyond about two waves per SIMD the extra instructions cost
-// more. Microseconds with 64 / 32 / 16 / 8 / 4 / 2 rays a wave: 1,009 rays
-// 46 / 39 / 33 / 29 / 28 / 28; 60,000 rays 116 / 96 / 110 / 113 / 123 / 142;
-// a 256x256 frame 75 / 70 / 71 / 71 / 72 / 90; 300,007 rays 152 / 177 / 216.
-uint32_t wave_rays_log2(uint64_t rays) {
-  uint32_t k = 2;
-  while (k < 6 && rays > (uint64_t(2048) << k)) ++k;
-  return k;
-}
-
 // Workgroups of a plain launch over n rays.
 dim3 wave_grid(uint32_t n, uint32_t rays_log2) {
   return dim3(static_cast<uint32_t>((static_cast<uint64_t>(n) + (1u << rays_log2) - 1u) >>
@@ -477,6 +463,20 @@ bool validate_desc(const svo_tree_desc& d, std::string* err) {
 }
 
 }  // namespace
+
+// log2 of the rays a wave of a plain launch takes: 64 once that makes 2048
+// waves (two per SIMD), fewer, down to 4, for smaller launches. Such a launch
+// lasts as long as its slowest wave, and a wave runs the paths of all its
+// lanes, so a chip with idle SIMDs answers sooner with its rays spread over
+// more waves; beyond about two waves per SIMD the extra instructions cost
+// more. Microseconds with 64 / 32 / 16 / 8 / 4 / 2 rays a wave: 1,009 rays
+// 46 / 39 / 33 / 29 / 28 / 28; 60,000 rays 116 / 96 / 110 / 113 / 123 / 142;
+// a 256x256 frame 75 / 70 / 71 / 71 / 72 / 90; 300,007 rays 152 / 177 / 216.
+uint32_t wave_rays_log2(uint64_t rays) {
+  uint32_t k = 2;
+  while (k < 6 && rays > (uint64_t(2048) << k)) ++k;
+  return k;
+}
 
 void timing_enable(bool on) { g_timing = on; }
 
