@@ -59,7 +59,7 @@ struct alignas(16) BatchJob {
   uint32_t tile_major;  // 1: outputs stored tile after tile from out[0]
   float viewing_distance;  // > 0: get_by_ray_at_lod with this distance
   uint32_t tiles_x_rcp;    // floor((2^32 - 1) / tiles_x), for tile_row
-  uint32_t pad;
+  uint32_t last_first;     // render: the per-tile kernel starts at the last row (looks_down)
   Camera cam;
   const float* rays;
   // cast jobs: the traversal order of the rays (lane k of the job's tiles
@@ -217,7 +217,9 @@ void batch_tile_kernel(const char* __restrict__ table, uint32_t njobs, uint32_t 
   const TreeView& tv = reinterpret_cast<const TreeView*>(table + trees_offset)[tree];
   if ((threadIdx.x >> rays_log2) != 0u) return;
   const uint32_t lane = ((blockIdx.x << rays_log2) & 63u) + threadIdx.x;
-  cast_tile<false, LOD, 8, 8>(job, tv, tile - job.tile_begin, lane, nullptr, 0u);
+  uint32_t local = tile - job.tile_begin;
+  if (job.last_first) local = job.tile_count - 1u - local;
+  cast_tile<false, LOD, 8, 8>(job, tv, local, lane, nullptr, 0u);
 }
 
 // LOD compiles in get_by_ray_at_lod for jobs with a viewing distance; a
@@ -454,6 +456,7 @@ int fill_job(BatchJob& j, const BatchJobIn& in, uint32_t ti, uint32_t tw, uint32
     j.first_tile = in.first_tile;
     j.tile_major = in.tile_major ? 1u : 0u;
     j.cam = in.cam;
+    j.last_first = looks_down(in.cam, in.width, in.height) ? 1u : 0u;
   } else {
     if (in.width && !in.rays) {
       *err = "cast job without rays";

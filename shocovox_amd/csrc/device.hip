@@ -57,18 +57,20 @@ __global__ __launch_bounds__(64) void cast_lod_kernel(TreeView t, const float* _
   store_result(t, out, i, res, o);
 }
 
-// A plain image kernel's tiles, one per workgroup in row order: 2^log_w x
-// 2^log_h pixels, one per lane. (The grid's second dimension only continues
-// the first, which holds fewer than 2^32 threads.)
+// A plain image kernel's tiles, one per workgroup in row order, from the last
+// row when `last_first`: 2^log_w x 2^log_h pixels, one per lane. (The grid's
+// second dimension only continues the first, which holds fewer than 2^32
+// threads.)
 struct Tiles {
-  uint32_t log_w, log_h, per_row, count;
+  uint32_t log_w, log_h, per_row, count, last_first;
 };
 
 // The pixel of this lane; false when it has none.
 __device__ inline bool tile_pixel(const Tiles& tl, uint32_t w, uint32_t h, uint32_t* x,
                                   uint32_t* y) {
-  const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
+  uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
   if (tile >= tl.count) return false;
+  if (tl.last_first) tile = tl.count - 1u - tile;
   const uint32_t ty = tile / tl.per_row, tx = tile - ty * tl.per_row;
   *x = (tx << tl.log_w) + (threadIdx.x & ((1u << tl.log_w) - 1u));
   *y = (ty << tl.log_h) + (threadIdx.x >> tl.log_w);
@@ -299,13 +301,16 @@ dim3 wave_grid(uint32_t n, uint32_t rays_log2) {
                                     rays_log2));
 }
 
-Tiles tiles_for(uint32_t w, uint32_t h) {
+Tiles tiles_for(uint32_t w, uint32_t h, bool last_first) {
   const uint32_t k = wave_rays_log2(static_cast<uint64_t>(w) * h);
   Tiles tl;
   tl.log_w = (k + 1u) / 2u;
   tl.log_h = k / 2u;
   tl.per_row = (w >> tl.log_w) + ((w & ((1u << tl.log_w) - 1u)) != 0u);
   tl.count = tl.per_row * ((h >> tl.log_h) + ((h & ((1u << tl.log_h) - 1u)) != 0u));
+  // (up to 8192 tiles start at once, eight on each of 1024 SIMDs: for them the
+  // order gains nothing; a 256x256 frame measured 70 us so and 71 reversed)
+  tl.last_first = last_first && tl.count > 8192u ? 1u : 0u;
   return tl;
 }
 // Grid of a plain image launch (w, h > 0, fewer than 2^32 pixels).
@@ -1077,7 +1082,7 @@ int device_render_lod(const DeviceTree& t, const Camera& cam, uint32_t w, uint32
   if (!image_fits(w, h, err)) return SVO_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
-  const Tiles tl = tiles_for(w, h);
+  const Tiles tl = tiles_for(w, h, looks_down(cam, w, h));
   hipLaunchKernelGGL(frame_lod_kernel, tile_grid(tl), dim3(64), 0, s, t.view, cam, w, h,
                      viewing_distance, tl, to_ptrs(out));
   hipError_t e = hipGetLastError();
@@ -1093,7 +1098,7 @@ int device_render(const DeviceTree& t, const Camera& cam, uint32_t w, uint32_t h
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
   if (g_render_variant == kAutoVariant) {
-    const Tiles tl = tiles_for(w, h);
+    const Tiles tl = tiles_for(w, h, looks_down(cam, w, h));
     hipLaunchKernelGGL(frame_kernel, tile_grid(tl), dim3(64), 0, s, t.view, cam, w, h, tl,
                        to_ptrs(out));
     const hipError_t e = hipGetLastError();
@@ -1156,7 +1161,7 @@ int device_render_rgba8(const DeviceTree& t, V3f origin, V3f dir, float glass_w,
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
-  const Tiles tl = tiles_for(w, h);
+  const Tiles tl = tiles_for(w, h, dir.y > 0.0f);  // (row 0 is the top here)
   if (convention == 0)
     hipLaunchKernelGGL(shade_kernel<0>, tile_grid(tl), dim3(64), 0, s, t.view, sp, w, h, tl,
                        out);

@@ -1201,4 +1201,17 @@ SVO_HD inline V3f camera_ray_dir(const Camera& c, uint32_t x, uint32_t y) {
   return normalized(glass - c.origin);
 }
 
+// Whether the camera looks down (or level): its image's top rows then hold the
+// rays nearest to the horizon, which graze the most content. A launch ends
+// with its slowest tiles, so the kernels that hand out an image's tiles in
+// order begin with those rows (row 0 is the bottom): 1080p caves frame 184 ->
+// 169 us, 4K heightfield frame 526 -> 503 us, eight 1080p frames in one run
+// 738 -> 714 us; 720p over spheres 145 -> 149 us. (An image drawn top row
+// first, begun at the bottom instead: 123 -> 125 us.)
+SVO_HD inline bool looks_down(const Camera& c, uint32_t w, uint32_t h) {
+  const float x = 0.5f * static_cast<float>(w) * c.pixel_w;
+  const float y = 0.5f * static_cast<float>(h) * c.pixel_h;
+  return !(c.bottom_left.y + c.right.y * x + c.up.y * y - c.origin.y > 0.0f);
+}
+
 }  // namespace svo
