@@ -163,3 +163,19 @@ def test_lod_rays_that_leave_the_content_behind(vd):
     rays = np.concatenate([rays, far])
     assert_parity(_oracle(t).cast(rays, viewing_distance=vd),
                   hostsim.cast(f, rays, viewing_distance=vd), f"vd={vd}")
+
+
+@pytest.mark.parametrize("vd", [2.0, 3.0, 7.0, 15.0, 40.0, 120.0])
+def test_mip_test_shortcut_near_its_margin(vd):
+    """mip_test answers without the exact distance when the level is clearly
+    high enough: viewing distances at which rays meet levels on both sides of
+    the test, close to and far from it, against the oracle."""
+    t = Octree.scene(2, 64, 4, 6)
+    t.albedo_mip_map_resampling_strategy().switch_albedo_mip_maps(True).recalculate_mips()
+    f = t.flatten().arrays()
+    rays = W.incoherent_rays(64, 1500, seed=9)
+    back = rays.copy()
+    back[:, :3] -= back[:, 3:] * np.linspace(0.0, 400.0, len(back), dtype=np.float32)[:, None]
+    rays = np.concatenate([rays, back])
+    assert_parity(_oracle(t).cast(rays, viewing_distance=vd),
+                  hostsim.cast(f, rays, viewing_distance=vd), f"vd={vd}")
