@@ -303,16 +303,17 @@ typedef struct svo_hits {
 } svo_hits;
 
 /* Octree::get_by_ray for n rays (src/raytracing/raytracing_on_cpu.rs:316-318).
- * rays: device array of n x {origin.xyz, direction.xyz} f32. From the
- * threshold of svo_cast_set_order_threshold up, the rays are traversed in the order of
- * (origin cell on a 64^3 grid of the tree, Morton order; direction octant),
- * found by a radix sort on `stream` with scratch from the stream-ordered
- * allocator; each ray's outputs are its own in any order. */
+ * rays: device array of n x {origin.xyz, direction.xyz} f32. Large
+ * arrays (from about 400,000 rays) are streamed: a wave's lanes take its rays
+ * one after another, in no fixed order; each ray's outputs are its own. */
 int svo_cast(const svo_tree* dtree, const float* rays, uint32_t n, const svo_hits* out,
              void* stream);
 /* No counterpart in the reference (a tuning knob): the ray count from which
- * svo_cast, svo_cast_at_lod and svo_batch_run's cast jobs order the rays (default
- * 2^20; 0 never orders; above 2^31 - 1 rays stay unordered). Process-wide.
+ * svo_cast, svo_cast_at_lod and svo_batch_run's cast jobs traverse the rays in the
+ * order of (origin cell on a 64^3 grid of the tree, Morton order; direction
+ * octant), found by a radix sort on the call's stream, instead of streaming
+ * them. At the default, 2^20, only the persistent batched variants do;
+ * 0 never orders; above 2^31 - 1 rays stay unordered. Process-wide.
  * The sort's scratch comes from the device's default memory pool, which is
  * set to keep freed memory for reuse; without device memory for the sort the
  * rays keep their own order. svo_batch_run_static never orders. */

@@ -511,6 +511,28 @@ hipError_t launch_tiles(const char* table, uint32_t n, uint64_t tiles, bool lod,
   return hipGetLastError();
 }
 
+// Job i of a per-tile run: like fill_job, but a large ray array keeps no tiles
+// and is listed in `streamed`, to run by its own launch (launch_cast_stream).
+// *all counts the tiles of both kinds.
+int fill_job_or_stream(BatchJob& j, const BatchJobIn& in, uint32_t i, uint32_t ti, bool per_tile,
+                       uint32_t tw, uint32_t th, uint64_t* tiles, uint64_t* all, bool* lod,
+                       std::vector<uint32_t>* streamed, std::string* err) {
+  const bool stream = per_tile && in.kind == 1 && in.rays &&
+                      streams_cast(in.width, in.viewing_distance > 0.0f);
+  bool job_lod = false;
+  const int st = fill_job(j, in, ti, tw, th, all, &job_lod, err);
+  if (st != SVO_OK) return st;
+  j.tile_begin = static_cast<uint32_t>(*tiles);
+  if (stream) {
+    j.tile_count = 0;
+    streamed->push_back(i);
+  } else {
+    *tiles += j.tile_count;
+    *lod = *lod || job_lod;
+  }
+  return SVO_OK;
+}
+
 }  // namespace
 
 struct BatchContext {
@@ -705,8 +727,10 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
   const size_t trees_offset = trees_offset_for(n);
   TreeView* trees = reinterpret_cast<TreeView*>(base + trees_offset);
   std::unordered_map<const void*, uint32_t> tree_index;
-  uint64_t tiles = 0;
+  const BatchVariant& v = kBatchVariants[b->variant];
+  uint64_t tiles = 0, all_tiles = 0;
   bool any_lod = false;
+  std::vector<uint32_t> streamed;
   for (uint32_t i = 0; i < n; ++i) {
     const BatchJobIn& in = jobs[i];
     if (!in.tree || in.tree->device != b->device) {
@@ -722,8 +746,8 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
     } else {
       ti = it->second;
     }
-    const int st = fill_job(out[i], in, ti, kBatchVariants[b->variant].tile_w,
-                            kBatchVariants[b->variant].tile_h, &tiles, &any_lod, err);
+    const int st = fill_job_or_stream(out[i], in, i, ti, v.per_tile, v.tile_w, v.tile_h, &tiles,
+                                      &all_tiles, &any_lod, &streamed, err);
     if (st != SVO_OK) return st;
   }
   // large cast jobs traverse their rays in svo_cast's order (kernels on `s`
@@ -733,7 +757,9 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
   if (kBatchVariants[b->variant].orders_casts)
     for (uint32_t i = 0; i < n; ++i) {
       const uint32_t threshold = cast_order_threshold();
-      if (jobs[i].kind != 1 || threshold == 0 || jobs[i].width < threshold) continue;
+      if (jobs[i].kind != 1 || threshold == 0 || jobs[i].width < threshold ||
+          (v.per_tile && streams_cast(jobs[i].width, jobs[i].viewing_distance > 0.0f)))
+        continue;
       uint32_t* ord = nullptr;
       const int st = order_rays(jobs[i].rays, jobs[i].width, jobs[i].tree->view.size, &ord, s, err);
       if (st == SVO_OUT_OF_DEVICE_MEMORY) continue;  // this job keeps its rays' own order
@@ -746,9 +772,9 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
       out[i].order = ord;
     }
   fill_header(base, n, tiles, trees_offset);
-  b->last_tiles = tiles;
+  b->last_tiles = all_tiles;
   const size_t used = trees_offset + tree_index.size() * sizeof(TreeView);
-  const bool per_tile = kBatchVariants[b->variant].per_tile;
+  const bool per_tile = v.per_tile;
   if (any_lod && !per_tile && !b->exec_lod) {
     const int st = build_graph(b, kBatchVariants[b->variant].lod_fn, &b->graph_lod,
                                &b->copy_node_lod, &b->exec_lod, err);
@@ -765,6 +791,16 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
     else if (e == hipSuccess)
       e = hipMemcpyAsync(b->dev, base, used, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = launch_tiles(static_cast<const char*>(b->dev), n, tiles, any_lod, s);
+    int st = SVO_OK;
+    for (size_t k = 0; k < streamed.size() && e == hipSuccess && st == SVO_OK; ++k) {
+      const BatchJobIn& in = jobs[streamed[k]];
+      st = launch_cast_stream(*in.tree, in.rays, in.width, in.viewing_distance,
+                              in.viewing_distance > 0.0f, in.out, s, err);
+    }
+    if (st != SVO_OK) {
+      for (uint32_t* p : orders) (void)hipFreeAsync(p, s);
+      return st;
+    }
   } else {
     hipGraphExec_t exec = any_lod ? b->exec_lod : b->exec;
     if (e == hipSuccess)
@@ -858,8 +894,10 @@ int run_static(const svo_job* jobs, uint32_t n, void* stream, std::string* err) 
   TreeView* trees = reinterpret_cast<TreeView*>(base + trees_offset);
   const DeviceTree* keys[kStaticMaxJobs];
   uint32_t ntrees = 0;
-  uint64_t tiles = 0;
+  const BatchVariant& v = kBatchVariants[g_batch_variant];
+  uint64_t tiles = 0, all_tiles = 0;
   bool any_lod = false;
+  std::vector<uint32_t> streamed;
   for (uint32_t i = 0; i < n; ++i) {
     const svo_job& j = jobs[i];
     if (!j.tree || !j.tree->dev || j.tree->dev->device != device) {
@@ -891,16 +929,21 @@ int run_static(const svo_job* jobs, uint32_t n, void* stream, std::string* err) 
       keys[ntrees++] = in.tree;
       trees[ti] = in.tree->view;
     }
-    st = fill_job(out[i], in, ti, kBatchVariants[g_batch_variant].tile_w,
-                  kBatchVariants[g_batch_variant].tile_h, &tiles, &any_lod, err);
+    st = fill_job_or_stream(out[i], in, i, ti, v.per_tile, v.tile_w, v.tile_h, &tiles, &all_tiles,
+                            &any_lod, &streamed, err);
     if (st != SVO_OK) return st;
   }
-  if (tiles == 0) return SVO_OK;  // nothing to cast, nothing to write
+  for (uint32_t i : streamed) {
+    const svo_job& j = jobs[i];
+    st = launch_cast_stream(*j.tree->dev, j.rays, j.width, j.viewing_distance,
+                            j.viewing_distance > 0.0f, j.out, stream, err);
+    if (st != SVO_OK) return st;
+  }
+  if (tiles == 0) return SVO_OK;  // nothing else to cast, nothing to write
   fill_header(base, n, tiles, trees_offset);
   const size_t used = trees_offset + ntrees * sizeof(TreeView);
   hipStream_t s = static_cast<hipStream_t>(stream);
   upload_table(sd->scratch, base, used, s);
-  const BatchVariant& v = kBatchVariants[g_batch_variant];
   if (v.per_tile) {
     (void)launch_tiles(sd->scratch, n, tiles, any_lod, s);
   } else {

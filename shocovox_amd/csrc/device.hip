@@ -57,6 +57,64 @@ __global__ __launch_bounds__(64) void cast_lod_kernel(TreeView t, const float* _
   store_result(t, out, i, res, o);
 }
 
+// A large ray array, mostly of rays that have little to do with each other:
+// each wave owns `per_wave` consecutive rays and its lanes take them one after
+// another. Neighbouring rays differ in length and in what each iteration does,
+// so a wave of one ray per lane has 7-14% of its lanes active on average. Two
+// things raise that: lanes whose ray has ended take the next rays as soon as
+// kRefill of them wait (results are stored and rays set up for them together),
+// and a lane walks at most kSlice brick cells per iteration, so that the others
+// do not wait for the longest walk of the wave (walk_iterate's slices).
+// (kSlice 2 / 4 / 6 / 8 / 16 on 3M rays: spheres 512^3 - / 873 / 822 / 818 /
+// 921 us, caves 512^3 967 / 877 / 895 / 975 / 1130; kRefill 16 and 32 measured
+// within 3% of 24.)
+constexpr int kSlice = 6;
+constexpr uint32_t kRefill = 24;
+template <bool LOD>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6)))
+void cast_stream_kernel(TreeView t, const float* __restrict__ rays, uint32_t n,
+                        float viewing_distance, uint32_t per_wave, HitPtrs out) {
+  uint64_t next = static_cast<uint64_t>(blockIdx.x) * per_wave;  // of the rays not yet taken
+  const uint64_t last = min(static_cast<uint64_t>(n), next + per_wave);
+  constexpr uint32_t kNone = 0xFFFFFFFFu;
+  uint32_t i = kNone;  // this lane's ray
+  V3f o{0.0f, 0.0f, 0.0f};
+  RayWalk w;
+  walk_begin<LOD>(t, o, V3f{1.0f, 1.0f, 1.0f}, w);
+  w.end = WALK_MISS;
+  // Ends: each pass either iterates a running ray (whose iterations are
+  // bounded), or stores and takes rays, of which there are finitely many.
+  for (;;) {
+    const uint64_t running = __ballot(w.end == WALK_RUNS);
+    const uint32_t idle = 64u - static_cast<uint32_t>(__popcll(running));
+    if (running == 0ull || (idle >= kRefill && next < last)) {
+      if (w.end != WALK_RUNS) {
+        if (i != kNone) {
+          const CastResult res = walk_result<LOD, true>(t, nullptr, 0u, w);
+          const float* r = rays + 6ull * i;
+          store_result(t, out, i, res, V3f{r[0], r[1], r[2]});
+        }
+        const uint64_t k =
+            next + __builtin_amdgcn_mbcnt_hi(
+                       static_cast<uint32_t>(~running >> 32),
+                       __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(~running), 0u));
+        i = kNone;
+        if (k < last) {
+          i = static_cast<uint32_t>(k);
+          const float* r = rays + 6ull * i;
+          o = V3f{r[0], r[1], r[2]};
+          walk_begin<LOD>(t, o, V3f{r[3], r[4], r[5]}, w);
+        }
+      }
+      next += idle;
+      if (running == 0ull && __ballot(i != kNone) == 0ull) break;
+      continue;
+    }
+    if (w.end == WALK_RUNS)
+      walk_iterate<LOD, true, kSlice>(t, t.ray_lut, o, nullptr, 0u, viewing_distance, w);
+  }
+}
+
 // A plain image kernel's tiles, one per workgroup in row order, from the last
 // row when `last_first`: 2^log_w x 2^log_h pixels, one per lane. (The grid's
 // second dimension only continues the first, which holds fewer than 2^32
@@ -1017,8 +1075,57 @@ void device_tree_destroy(DeviceTree* t) {
   delete t;
 }
 
-int device_cast(const DeviceTree& t, const float* rays, uint32_t n, const svo_hits& out,
-                void* stream, std::string* err) {
+namespace {
+// Ray count from which casts are ordered (set_cast_order_threshold). Left at
+// the default, plain and per-tile launches stream large casts instead.
+constexpr uint32_t kDefaultOrderThreshold = 1u << 20;
+std::atomic<uint32_t> g_cast_order_threshold{kDefaultOrderThreshold};
+// The threshold where a caller chose one, else 0.
+uint32_t chosen_order_threshold() {
+  const uint32_t n = g_cast_order_threshold.load();
+  return n == kDefaultOrderThreshold ? 0u : n;
+}
+
+// Waves of a streamed cast: as many as run at once at six waves per SIMD.
+constexpr uint32_t kStreamWaves = 6 * 1024;
+}  // namespace
+
+void set_cast_order_threshold(uint32_t n) { g_cast_order_threshold.store(n); }
+uint32_t cast_order_threshold() { return g_cast_order_threshold.load(); }
+
+// More rays than lanes run at once: from there on a lane has further rays to
+// take. 3M rays in their own order, streamed against one ray per lane ordered
+// by origin and direction (order.hip; its sort is 0.2 ms): spheres 512^3 0.82
+// against 1.20 ms, caves 512^3 0.90 against 1.37; 1.2M rays, caves 0.44
+// against 0.69; one ray per lane unordered: 1.42, 1.18 and 0.54 ms. Around the
+// line: 300,007 rays 188 streamed, 152 us one per lane; 500,000 rays 233 and
+// 245 us.
+// LOD rays end sooner and gain less, so for them the line is twice as far:
+// 500,009 rays 196 us streamed, 184 one per lane; 1M rays 291 and 295; 3M into
+// a 256^3 heightfield 715 and 999.
+bool streams_cast(uint64_t n, bool lod) {
+  const uint32_t order_from = chosen_order_threshold();
+  return n > uint64_t(kStreamWaves) * (lod ? 128u : 64u) && (order_from == 0u || n < order_from);
+}
+
+int launch_cast_stream(const DeviceTree& t, const float* rays, uint32_t n, float viewing_distance,
+                       bool lod, const svo_hits& out, void* stream, std::string* err) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const uint32_t per = (n - 1u) / kStreamWaves + 1u;
+  const dim3 grid((n - 1u) / per + 1u);
+  if (lod)
+    hipLaunchKernelGGL(cast_stream_kernel<true>, grid, dim3(64), 0, s, t.view, rays, n,
+                       viewing_distance, per, to_ptrs(out));
+  else
+    hipLaunchKernelGGL(cast_stream_kernel<false>, grid, dim3(64), 0, s, t.view, rays, n,
+                       viewing_distance, per, to_ptrs(out));
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? SVO_OK : hip_fail(e, "cast_stream_kernel launch", err);
+}
+
+namespace {
+int cast_any(const DeviceTree& t, const float* rays, uint32_t n, float viewing_distance, bool lod,
+             const svo_hits& out, void* stream, std::string* err) {
   if (n == 0) return SVO_OK;
   if (rays == nullptr) {
     *err = "rays is NULL";
@@ -1026,53 +1133,41 @@ int device_cast(const DeviceTree& t, const float* rays, uint32_t n, const svo_hi
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
+  if (streams_cast(n, lod)) {
+    const int st = launch_cast_stream(t, rays, n, viewing_distance, lod, out, stream, err);
+    if (st == SVO_OK) timer.done();
+    return st;
+  }
   uint32_t* order = nullptr;
-  const uint32_t threshold = cast_order_threshold();
+  const uint32_t threshold = chosen_order_threshold();
   if (threshold != 0 && n >= threshold) {
     // without device memory for the sort the rays keep their own order
     const int st = order_rays(rays, n, t.view.size, &order, s, err);
     if (st != SVO_OK && st != SVO_OUT_OF_DEVICE_MEMORY) return st;
   }
   const uint32_t k = wave_rays_log2(n);
-  hipLaunchKernelGGL(cast_kernel, wave_grid(n, k), dim3(64), 0, s, t.view, rays, n, order, k,
-                     to_ptrs(out));
-  hipError_t e = hipGetLastError();
+  if (lod)
+    hipLaunchKernelGGL(cast_lod_kernel, wave_grid(n, k), dim3(64), 0, s, t.view, rays, n,
+                       viewing_distance, order, k, to_ptrs(out));
+  else
+    hipLaunchKernelGGL(cast_kernel, wave_grid(n, k), dim3(64), 0, s, t.view, rays, n, order, k,
+                       to_ptrs(out));
+  const hipError_t e = hipGetLastError();
   if (order) (void)hipFreeAsync(order, s);
-  if (e != hipSuccess) return hip_fail(e, "cast_kernel launch", err);
+  if (e != hipSuccess) return hip_fail(e, lod ? "cast_lod_kernel launch" : "cast_kernel launch", err);
   timer.done();
   return SVO_OK;
 }
-
-namespace {
-std::atomic<uint32_t> g_cast_order_threshold{1u << 20};
 }  // namespace
 
-void set_cast_order_threshold(uint32_t n) { g_cast_order_threshold.store(n); }
-uint32_t cast_order_threshold() { return g_cast_order_threshold.load(); }
+int device_cast(const DeviceTree& t, const float* rays, uint32_t n, const svo_hits& out,
+                void* stream, std::string* err) {
+  return cast_any(t, rays, n, 0.0f, false, out, stream, err);
+}
 
 int device_cast_lod(const DeviceTree& t, const float* rays, uint32_t n, float viewing_distance,
                     const svo_hits& out, void* stream, std::string* err) {
-  if (n == 0) return SVO_OK;
-  if (rays == nullptr) {
-    *err = "rays is NULL";
-    return SVO_INVALID_ARGUMENT;
-  }
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  LaunchTimer timer(s);
-  uint32_t* order = nullptr;
-  const uint32_t threshold = cast_order_threshold();
-  if (threshold != 0 && n >= threshold) {
-    const int st = order_rays(rays, n, t.view.size, &order, s, err);
-    if (st != SVO_OK && st != SVO_OUT_OF_DEVICE_MEMORY) return st;
-  }
-  const uint32_t k = wave_rays_log2(n);
-  hipLaunchKernelGGL(cast_lod_kernel, wave_grid(n, k), dim3(64), 0, s, t.view, rays, n,
-                     viewing_distance, order, k, to_ptrs(out));
-  hipError_t e = hipGetLastError();
-  if (order) (void)hipFreeAsync(order, s);
-  if (e != hipSuccess) return hip_fail(e, "cast_lod_kernel launch", err);
-  timer.done();
-  return SVO_OK;
+  return cast_any(t, rays, n, viewing_distance, true, out, stream, err);
 }
 
 int device_render_lod(const DeviceTree& t, const Camera& cam, uint32_t w, uint32_t h,

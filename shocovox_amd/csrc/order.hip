@@ -1,6 +1,8 @@
-// Traversal order of a large ray array (svo_cast). Rays whose origins lie
+// Traversal order of a large ray array, for the persistent batched variants and
+// for callers that ask svo_cast for it (set_cast_order_threshold); by default
+// svo_cast streams such arrays, which needs no sort. Rays whose origins lie
 // close together and whose directions share an octant walk the same nodes
-// and bricks, so svo_cast traverses them side by side: each ray gets the key
+// and bricks, so they are traversed side by side: each ray gets the key
 // (Morton code of its origin on a 64^3 grid over the tree) * 8 + (direction
 // octant), a stable radix sort of the keys gives the order, and the cast
 // kernel's lane i traverses ray order[i] and writes that ray's own outputs.

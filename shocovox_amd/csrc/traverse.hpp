@@ -249,11 +249,18 @@ SVO_HD inline uint32_t bitmap_cell(V3f bp) {
 // traverse_brick (raytracing_on_cpu.rs:156-252) over the occupancy of Parted
 // brick `word` with bounds bb: moves p to where the walk ends and returns
 // whether that is in an occupied cell, whose flat index goes to *cell.
-template <bool P2>
+// With SLICE > 0 (P2 only) a call takes at most SLICE steps; a walk that has
+// not ended by then leaves its cell in *cell and sets *more, and the next call
+// goes on from there (a cell's far corner is the same value whether it is
+// reached by steps or formed from the cell's index).
+constexpr uint32_t NO_CELL = 0xFFFFFFFFu;
+template <bool P2, int SLICE = 0>
 SVO_HD __attribute__((always_inline)) inline bool walk_brick(const TreeView& t, uint32_t word,
                                                              Cube bb, V3f d, V3f sig, V3f scale,
                                                              V3f* p, uint32_t* cell,
-                                                             uint32_t* flags) {
+                                                             uint32_t* flags,
+                                                             bool* more = nullptr) {
+  static_assert(P2 || SLICE == 0, "only the P2 form walks in slices");
   const int dim = static_cast<int>(t.dim);
   const float fdim = static_cast<float>(t.dim);
   const float rcp_size = size_rcp<P2>(bb.size);
@@ -273,6 +280,12 @@ SVO_HD __attribute__((always_inline)) inline bool walk_brick(const TreeView& t, 
   int ix = clampi(f2i32(pib.x));
   int iy = clampi(f2i32(pib.y));
   int iz = clampi(f2i32(pib.z));
+  if (SLICE > 0 && *cell != NO_CELL) {
+    const uint32_t k = static_cast<uint32_t>(__builtin_ctz(t.dim));
+    ix = static_cast<int>(*cell & (t.dim - 1u));
+    iy = static_cast<int>((*cell >> k) & (t.dim - 1u));
+    iz = static_cast<int>(*cell >> (2u * k));
+  }
   const float unit = div_size<P2>(bb.size, fdim, t.inv_dim);
   // A step moves the cell by signum(direction) on the axes that stepped and
   // leaves the others (their step component is +0.0, and cell corners are
@@ -329,9 +342,9 @@ SVO_HD __attribute__((always_inline)) inline bool walk_brick(const TreeView& t, 
     // run 1.09 -> 0.97 ms.
     uint32_t flat = (ax | (ay << shift) | (az << (2u * shift))) ^ mirror;
     uint32_t bits = occ_word(t, occ_off, flat, true);
-    uint32_t bit;
+    uint32_t bit, stop;
     float m;
-    for (;;) {
+    for (int left = SLICE;;) {
       bool sx, sy, sz;
       V3f q = *p;
       m = dda_step_far(d, &q, cmin, scale, &sx, &sy, &sz);
@@ -358,16 +371,23 @@ SVO_HD __attribute__((always_inline)) inline bool walk_brick(const TreeView& t, 
       // so the cell leaves the brick within 3 dim steps. A NaN step moves
       // nothing (p becomes NaN and stays so), so the loop would repeat that
       // state: it ends here.
-      const uint32_t stop = bit | (axes & ~dm1);
+      stop = bit | (axes & ~dm1);
       if ((stop != 0u) | !(m == m)) break;
+      if (SLICE > 0 && --left == 0) break;
     }
 #if defined(__HIP_DEVICE_COMPILE__)
-    // (opaque here, so that the two tests below are made after the loop and
-    // not carried through it as masks)
-    asm volatile("" : "+v"(bit), "+v"(m));
+    // (opaque here, so that the tests below are made after the loop and not
+    // carried through it as masks)
+    asm volatile("" : "+v"(bit), "+v"(m), "+v"(stop));
 #endif
     occupied = bit != 0u;
     in = !(m == m);
+    if (SLICE > 0) {
+      *more = (stop == 0u) & (m == m);
+      *cell = flat;
+      if (in && !occupied) *flags |= FLAG_ITERATION_GUARD;
+      return occupied;
+    }
     ix = static_cast<int>(flat & dm1);
     iy = static_cast<int>((flat >> shift) & dm1);
     iz = static_cast<int>(flat >> (2u * shift));
@@ -586,248 +606,292 @@ struct RingStack {
 // Together a lone ray's iteration takes 0.56 us instead of 0.78, 8 1080p
 // frames in one batched run 0.90 ms instead of 0.96, one of them 0.185 ms
 // instead of 0.208.
-template <bool LOD, bool P2, class LutT>
-SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
-    const TreeView& t, const LutT* __restrict__ lut, V3f o, V3f d, const NodeRec* top,
-    uint32_t ntop, float viewing_distance) {
-  CastResult r;
-  r.hit = 0;
-  r.flags = 0;
+struct RayWalk {
+  V3f d, scale, p;
+  Cube bounds;
+  uint32_t target;
+  RingStack stk;
+  uint32_t dir_idx;  // hash_direction(d)
+  uint32_t neg;      // octant bits of the axes the ray runs backwards along
+  uint32_t steps, flags;
+  uint32_t cell;     // flat cell of a hit, or of a sliced walk that goes on (else NO_CELL)
+  uint32_t end;      // WALK_*
+  float mip_level;   // LOD
+};
+enum : uint32_t {
+  WALK_RUNS = 0,
+  WALK_HIT = 1,
+  WALK_HIT_MIP = 2,
+  WALK_MISS = 3,
+  WALK_GUARD = 4,
+  WALK_CRAWL = 5
+};
 
-  const V3f scale = dda_scale_factors(d);
-  const uint32_t dir_idx = hash_direction(d);
-  // the axes the ray runs backwards along (for a NaN component every scale
-  // factor is NaN and no step moves any axis)
-  const uint32_t neg =
-      octant_of(__builtin_signbit(d.x), __builtin_signbit(d.y), __builtin_signbit(d.z));
-  const Cube root{v3u(0.0f), t.size};
+template <bool LOD>
+SVO_HD __attribute__((always_inline)) inline void walk_begin(const TreeView& t, V3f o, V3f d,
+                                                            RayWalk& w) {
+  w.d = d;
+  w.scale = dda_scale_factors(d);
+  w.dir_idx = hash_direction(d);
+  // (for a NaN component every scale factor is NaN and no step moves any axis)
+  w.neg = octant_of(__builtin_signbit(d.x), __builtin_signbit(d.y), __builtin_signbit(d.z));
+  w.bounds = Cube{v3u(0.0f), t.size};
+  w.stk = RingStack{0u, 0u, 0u, 0u, 1u};  // the root pushed
+  float tt = 0.0f;
+  const int ir = intersect_ray(w.bounds, o, d, &tt);
+  w.p = ir != 0 ? o + d * (ir == 2 ? tt : 0.0f) : o;
+  w.target = hash_region(w.p - w.bounds.min, w.bounds.size / 2.0f);
+  w.steps = 0;
+  w.flags = 0;
+  w.cell = NO_CELL;
+  w.end = ir != 0 ? WALK_RUNS : WALK_MISS;
+  // log2(size / dim) of two powers of two, exactly
+  w.mip_level =
+      LOD ? static_cast<float>(__builtin_ctz(static_cast<uint32_t>(t.size) / t.dim)) : 0.0f;
+}
+
+// One iteration of the reference's stack loop and, when the stack has
+// emptied, its restart from the root (which ends the ray when the nudged point
+// leaves the tree). With SLICE > 0 a brick walk takes at most SLICE steps in
+// one call, and the calls that carry it on are not iterations.
+template <bool LOD, bool P2, int SLICE, class LutT>
+SVO_HD __attribute__((always_inline)) inline void walk_iterate(
+    const TreeView& t, const LutT* __restrict__ lut, V3f o, const NodeRec* top, uint32_t ntop,
+    float viewing_distance, RayWalk& w) {
   const float lo = 0.00001f;
   const float hi = 4.0f - 0.00001f;
-
-  RingStack stk{0u, 0u, 0u, 0u, 1u};  // the root pushed
-  Cube bounds = root;
-  V3f p;
-  uint32_t target;
-  {
-    float tt = 0.0f;
-    const int ir = intersect_ray(root, o, d, &tt);
-    if (ir != 0) {
-      p = o + d * (ir == 2 ? tt : 0.0f);
-      target = hash_region(p - root.min, root.size / 2.0f);
-    } else {
-      p = o;
-      target = OOB_OCTANT;
-    }
-  }
-  if (target == OOB_OCTANT) return miss_flags(0u);
-  uint32_t steps = 0;
-  uint32_t cell = 0;  // flat cell of a hit in a Parted brick
-  // log2(size / dim) of two powers of two, exactly
-  float mip_level =
-      LOD ? static_cast<float>(__builtin_ctz(static_cast<uint32_t>(t.size) / t.dim)) : 0.0f;
-  enum : uint32_t { RUNS = 0, HIT = 1, HIT_MIP = 2, MISS = 3, GUARD = 4, CRAWL = 5 };
-  uint32_t end = RUNS;
-  // One loop runs the reference's two: an iteration of its stack loop, and
-  // when the stack has emptied, its restart from the root (which ends the ray
-  // when the nudged point leaves the tree).
-  do {
-    // signum(d) per axis, formed again in every iteration from d's sign bits
-    // (one instruction each) rather than kept in three registers: the empty
-    // asm makes d opaque here, so the compiler cannot hoist these (or other
-    // values derived from d) out of the loop. For a NaN component the
-    // reference's signum is NaN and this one +-1; then every scale factor is
-    // NaN (each involves all three components), every DDA distance is NaN
-    // and no step selects a signum, so the difference is never observed.
+  V3f& d = w.d;
+  V3f& p = w.p;
+  const V3f scale = w.scale;
+  const uint32_t dir_idx = w.dir_idx, neg = w.neg;
+  Cube& bounds = w.bounds;
+  uint32_t& target = w.target;
+  RingStack& stk = w.stk;
+  uint32_t& steps = w.steps;
+  uint32_t& end = w.end;
+  // signum(d) per axis, formed again in every iteration from d's sign bits
+  // (one instruction each) rather than kept in three registers: the empty
+  // asm makes d opaque here, so the compiler cannot hoist these (or other
+  // values derived from d) out of the loop. For a NaN component the
+  // reference's signum is NaN and this one +-1; then every scale factor is
+  // NaN (each involves all three components), every DDA distance is NaN
+  // and no step selects a signum, so the difference is never observed.
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z));
+  asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z));
 #endif
-    V3f sig{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
-    ++steps;  // (against the bound at the iteration's end)
-    const uint32_t key = stk.s0;
-    const NodeRec& n = (key < ntop ? top : t.nodes)[key];
-    const uint64_t occ = n.occ;
-    const uint32_t meta = n.meta;
-    // the child word of the current target, read together with the header
-    // (same record, one round trip); with target OOB_OCTANT it is child[0]
-    // and unused
-    const uint32_t tword = n.child[target & 7u];
-    // the position in the node's 4x4x4 bitmap; the clamp to [lo, hi]
-    // (:425-436) is applied to the float position only where ADVANCE
-    // continues from it, the cell index comes from bitmap_cell
-    const float rcp_size = size_rcp<P2>(bounds.size);
-    V3f bp = bitmap_pos<P2>(p, bounds, rcp_size);
-    uint64_t ahead = lut[bitmap_cell(bp) * 8u + dir_idx];
-    auto moved_by_probe = [&]() {
-      bp = bitmap_pos<P2>(p, bounds, rcp_size);
-      ahead = lut[bitmap_cell(bp) * 8u + dir_idx];
+  V3f sig{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
+  const bool fresh = SLICE == 0 || w.cell == NO_CELL;
+  if (fresh) ++steps;  // (against the bound at the iteration's end)
+  bool more = false;
+  const uint32_t key = stk.s0;
+  const NodeRec& n = (key < ntop ? top : t.nodes)[key];
+  const uint64_t occ = n.occ;
+  const uint32_t meta = n.meta;
+  // the child word of the current target, read together with the header
+  // (same record, one round trip); with target OOB_OCTANT it is child[0]
+  // and unused
+  const uint32_t tword = n.child[target & 7u];
+  // the position in the node's 4x4x4 bitmap; the clamp to [lo, hi]
+  // (:425-436) is applied to the float position only where ADVANCE
+  // continues from it, the cell index comes from bitmap_cell
+  const float rcp_size = size_rcp<P2>(bounds.size);
+  V3f bp = bitmap_pos<P2>(p, bounds, rcp_size);
+  uint64_t ahead = lut[bitmap_cell(bp) * 8u + dir_idx];
+  auto moved_by_probe = [&]() {
+    bp = bitmap_pos<P2>(p, bounds, rcp_size);
+    ahead = lut[bitmap_cell(bp) * 8u + dir_idx];
 #if defined(__HIP_DEVICE_COMPILE__)
-      // (used here, so that the two requests are not merged into one after
-      // the probe)
-      asm volatile("" : "+v"(ahead));
+    // (used here, so that the two requests are not merged into one after
+    // the probe)
+    asm volatile("" : "+v"(ahead));
 #endif
-    };
-    const uint32_t kind = node_kind(meta);
-    const bool uniform = kind == KIND_UNIFORM_LEAF;  // backtracks after its probe
-    if (LOD && t.mips_enabled) {
-      if (mip_test(t, o, p, mip_level, viewing_distance)) {
-        if (n.mip == FORM_SOLID) end = HIT_MIP;
-        if (n.mip == FORM_PARTED) {
-          if (walk_brick<P2>(t, n.mip_word, bounds, d, sig, scale, &p, &cell, &r.flags))
-            end = HIT_MIP;
-          moved_by_probe();
-        }
-      }
-    }
-    if ((!LOD || end == RUNS) && target != OOB_OCTANT &&
-        (kind == KIND_UNIFORM_LEAF || kind == KIND_LEAF)) {
-      const uint32_t slot = uniform ? 0u : target;
-      const uint32_t form = brick_form(meta, slot);
-      if (form == FORM_SOLID) end = HIT;
-      if (form == FORM_PARTED) {
-        if (walk_brick<P2>(t, slot == target ? tword : n.child[0],
-                           uniform ? bounds : child_bounds_for(bounds, target), d, sig, scale,
-                           &p, &cell, &r.flags))
-          end = HIT;
+  };
+  const uint32_t kind = node_kind(meta);
+  const bool uniform = kind == KIND_UNIFORM_LEAF;  // backtracks after its probe
+  if (LOD && t.mips_enabled && fresh) {
+    if (mip_test(t, o, p, w.mip_level, viewing_distance)) {
+      if (n.mip == FORM_SOLID) end = WALK_HIT_MIP;
+      if (n.mip == FORM_PARTED) {
+        if (walk_brick<P2>(t, n.mip_word, bounds, d, sig, scale, &p, &w.cell, &w.flags))
+          end = WALK_HIT_MIP;
         moved_by_probe();
       }
     }
-    // signum(d) formed again past the probe, so that the values formed
-    // before it are dead inside the probe's DDA loop (whose registers then
-    // hold the per-axis cell moves rather than recomputing them each step)
+  }
+  if ((!LOD || end == WALK_RUNS) && target != OOB_OCTANT &&
+      (kind == KIND_UNIFORM_LEAF || kind == KIND_LEAF)) {
+    const uint32_t slot = uniform ? 0u : target;
+    const uint32_t form = brick_form(meta, slot);
+    if (form == FORM_SOLID) end = WALK_HIT;
+    if (form == FORM_PARTED) {
+      if (walk_brick<P2, SLICE>(t, slot == target ? tword : n.child[0],
+                         uniform ? bounds : child_bounds_for(bounds, target), d, sig, scale,
+                         &p, &w.cell, &w.flags, &more))
+        end = WALK_HIT;
+      if (SLICE > 0 && end == WALK_RUNS && !more) w.cell = NO_CELL;
+      moved_by_probe();
+    }
+  }
+  // signum(d) formed again past the probe, so that the values formed
+  // before it are dead inside the probe's DDA loop (whose registers then
+  // hold the per-axis cell moves rather than recomputing them each step)
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z), "+v"(end));
+  asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z), "+v"(end));
 #endif
-    if (end == RUNS) {
-      sig = V3f{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
-      // (an empty bitmap has nothing ahead)
-      const bool pop = uniform | (target == OOB_OCTANT) | ((occ & ahead) == 0ull);
-      Cube tb = child_bounds_for(bounds, target);
-      const bool push = !pop & (kind == KIND_INTERNAL) &
-                        ((occ & octant_bitmap_mask(target)) != 0ull) & (tword != INVALID_INDEX);
-      const bool emptied = pop & (stk.count == 1u);
-      // PUSH, POP and ADVANCE leave the next bounds and target here, and the
-      // stack moves once after them, by selects: the loop's state stays in
-      // the same registers on every path.
-      Cube next_bounds = bounds;
-      uint32_t next_target = target;
-      if (push) {
-        // PUSH (:484-492)
-        next_bounds = tb;
-        next_target = hash_region(p - tb.min, tb.size / 2.0f);
-      } else {
-        // POP (:445-475) and ADVANCE (:497-544) both begin with one DDA step,
-        // out of the node (POP, unless the stack empties) or out of the
-        // target child (ADVANCE); it is issued once for the lanes of both.
-        // (The POP's other values depend on the bounds only, so taking the
-        // step before them changes nothing; nor does a step taken by an
-        // ADVANCE that then meets the iteration bound, which ends the ray as
-        // a miss.)
-        bool sx = false, sy = false, sz = false;
-        if (!emptied)
-          dda_step_axes(d, sig, &p, (pop ? bounds : tb).min, (pop ? bounds : tb).size, scale, &sx,
-                        &sy, &sz);
-        const uint32_t moved = octant_of(sx, sy, sz);
-        if (pop) {
-          if (emptied) {
-            if (key == 0u && !uniform && target != OOB_OCTANT && kind != KIND_LEAF &&
-                (!LOD || !t.mips_enabled || n.mip == FORM_EMPTY ||
-                 mip_test_over(t, o, mip_level, viewing_distance))) {
-              end = CRAWL;
-            } else {
-              // the reference's restart from the root (:551-562), which ends
-              // the ray once the nudged point has left the tree (taken here,
-              // not at the next iteration's start: nothing happens in
-              // between)
-              p = p + d * 0.1f;
-              const bool inside = (p.x < t.size) & (p.y < t.size) & (p.z < t.size) &
-                                  (p.x > 0.0f) & (p.y > 0.0f) & (p.z > 0.0f);
-              next_target = hash_region(p, t.size / 2.0f);
-              next_bounds = root;
-              end = inside ? RUNS : MISS;
-            }
+  if ((SLICE == 0 || !more) && end == WALK_RUNS) {
+    sig = V3f{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
+    // (an empty bitmap has nothing ahead)
+    const bool pop = uniform | (target == OOB_OCTANT) | ((occ & ahead) == 0ull);
+    Cube tb = child_bounds_for(bounds, target);
+    const bool push = !pop & (kind == KIND_INTERNAL) &
+                      ((occ & octant_bitmap_mask(target)) != 0ull) & (tword != INVALID_INDEX);
+    const bool emptied = pop & (stk.count == 1u);
+    // PUSH, POP and ADVANCE leave the next bounds and target here, and the
+    // stack moves once after them, by selects: the loop's state stays in
+    // the same registers on every path.
+    Cube next_bounds = bounds;
+    uint32_t next_target = target;
+    if (push) {
+      // PUSH (:484-492)
+      next_bounds = tb;
+      next_target = hash_region(p - tb.min, tb.size / 2.0f);
+    } else {
+      // POP (:445-475) and ADVANCE (:497-544) both begin with one DDA step,
+      // out of the node (POP, unless the stack empties) or out of the
+      // target child (ADVANCE); it is issued once for the lanes of both.
+      // (The POP's other values depend on the bounds only, so taking the
+      // step before them changes nothing; nor does a step taken by an
+      // ADVANCE that then meets the iteration bound, which ends the ray as
+      // a miss.)
+      bool sx = false, sy = false, sz = false;
+      if (!emptied)
+        dda_step_axes(d, sig, &p, (pop ? bounds : tb).min, (pop ? bounds : tb).size, scale, &sx,
+                      &sy, &sz);
+      const uint32_t moved = octant_of(sx, sy, sz);
+      if (pop) {
+        if (emptied) {
+          if (key == 0u && !uniform && target != OOB_OCTANT && kind != KIND_LEAF &&
+              (!LOD || !t.mips_enabled || n.mip == FORM_EMPTY ||
+               mip_test_over(t, o, w.mip_level, viewing_distance))) {
+            end = WALK_CRAWL;
           } else {
-            // the parent's bounds and the sibling the step leads to
-            const float s2 = bounds.size * 2.0f;
-            const float rcp_s2 = size_rcp<P2>(s2);
-            const V3f pmin{sub_fmod_size<P2>(bounds.min.x, s2, rcp_s2),
-                           sub_fmod_size<P2>(bounds.min.y, s2, rcp_s2),
-                           sub_fmod_size<P2>(bounds.min.z, s2, rcp_s2)};
-            next_target = step_octant_moved(pop_octant<P2>(bounds, pmin), moved, neg);
-            next_bounds = Cube{pmin, s2};
+            // the reference's restart from the root (:551-562), which ends
+            // the ray once the nudged point has left the tree (taken here,
+            // not at the next iteration's start: nothing happens in
+            // between)
+            p = p + d * 0.1f;
+            const bool inside = (p.x < t.size) & (p.y < t.size) & (p.z < t.size) &
+                                (p.x > 0.0f) & (p.y > 0.0f) & (p.z > 0.0f);
+            next_target = hash_region(p, t.size / 2.0f);
+            next_bounds = Cube{v3u(0.0f), t.size};
+            end = inside ? WALK_RUNS : WALK_MISS;
           }
         } else {
-          // the rest of ADVANCE
-          next_target = step_octant_moved(target, moved, neg);
-          if (++steps > t.max_steps) end = GUARD;
-          bp = V3f{rclamp(bp.x, lo, hi), rclamp(bp.y, lo, hi), rclamp(bp.z, lo, hi)};
-          V3f move = bitmap_move<P2>(
-              V3f{sx ? sig.x : 0.0f, sy ? sig.y : 0.0f, sz ? sig.z : 0.0f}, bounds.size,
-              rcp_size);
-          bool on = (next_target != OOB_OCTANT) & (end == RUNS);
-          while (on) {
-            tb = child_bounds_for(bounds, next_target);
-            bp = bp + move;
-            // stop at a reachable occupied child or a non-empty leaf brick;
-            // both words are requested together, whichever the test needs
-            const uint64_t there = lut[bitmap_index(bp, &r.flags) * 8u + dir_idx];
-            const uint32_t word = n.child[next_target];
-            const bool child = (kind == KIND_INTERNAL) &
-                               ((occ & octant_bitmap_mask(next_target)) != 0ull) &
-                               ((there & occ) != 0ull) & (word != INVALID_INDEX);
-            const bool brick =
-                (kind == KIND_LEAF) & (brick_form(meta, next_target) != FORM_EMPTY);
-            on = false;
-            if (!(child | brick)) {
-              if (++steps > t.max_steps) end = GUARD;
-              dda_step_axes(d, sig, &p, tb.min, tb.size, scale, &sx, &sy, &sz);
-              move = bitmap_move<P2>(
-                  V3f{sx ? sig.x : 0.0f, sy ? sig.y : 0.0f, sz ? sig.z : 0.0f}, bounds.size,
-                  rcp_size);
-              next_target = step_octant_moved(next_target, octant_of(sx, sy, sz), neg);
-              on = (next_target != OOB_OCTANT) & (end == RUNS);
-            }
+          // the parent's bounds and the sibling the step leads to
+          const float s2 = bounds.size * 2.0f;
+          const float rcp_s2 = size_rcp<P2>(s2);
+          const V3f pmin{sub_fmod_size<P2>(bounds.min.x, s2, rcp_s2),
+                         sub_fmod_size<P2>(bounds.min.y, s2, rcp_s2),
+                         sub_fmod_size<P2>(bounds.min.z, s2, rcp_s2)};
+          next_target = step_octant_moved(pop_octant<P2>(bounds, pmin), moved, neg);
+          next_bounds = Cube{pmin, s2};
+        }
+      } else {
+        // the rest of ADVANCE
+        next_target = step_octant_moved(target, moved, neg);
+        if (++steps > t.max_steps) end = WALK_GUARD;
+        bp = V3f{rclamp(bp.x, lo, hi), rclamp(bp.y, lo, hi), rclamp(bp.z, lo, hi)};
+        V3f move = bitmap_move<P2>(
+            V3f{sx ? sig.x : 0.0f, sy ? sig.y : 0.0f, sz ? sig.z : 0.0f}, bounds.size,
+            rcp_size);
+        bool on = (next_target != OOB_OCTANT) & (end == WALK_RUNS);
+        while (on) {
+          tb = child_bounds_for(bounds, next_target);
+          bp = bp + move;
+          // stop at a reachable occupied child or a non-empty leaf brick;
+          // both words are requested together, whichever the test needs
+          const uint64_t there = lut[bitmap_index(bp, &w.flags) * 8u + dir_idx];
+          const uint32_t word = n.child[next_target];
+          const bool child = (kind == KIND_INTERNAL) &
+                             ((occ & octant_bitmap_mask(next_target)) != 0ull) &
+                             ((there & occ) != 0ull) & (word != INVALID_INDEX);
+          const bool brick =
+              (kind == KIND_LEAF) & (brick_form(meta, next_target) != FORM_EMPTY);
+          on = false;
+          if (!(child | brick)) {
+            if (++steps > t.max_steps) end = WALK_GUARD;
+            dda_step_axes(d, sig, &p, tb.min, tb.size, scale, &sx, &sy, &sz);
+            move = bitmap_move<P2>(
+                V3f{sx ? sig.x : 0.0f, sy ? sig.y : 0.0f, sz ? sig.z : 0.0f}, bounds.size,
+                rcp_size);
+            next_target = step_octant_moved(next_target, octant_of(sx, sy, sz), neg);
+            on = (next_target != OOB_OCTANT) & (end == WALK_RUNS);
           }
         }
       }
-      // PUSH shifts the stack down (its oldest entry drops out once four are
-      // held), POP shifts it up, and a POP that empties it is followed by the
-      // restart's push of the root; ADVANCE leaves it
-      const uint32_t s0 = stk.s0, s1 = stk.s1, s2 = stk.s2, s3 = stk.s3;
-      stk.s0 = push ? tword : (pop ? (emptied ? 0u : s1) : s0);
-      stk.s1 = push ? s0 : (pop ? s2 : s1);
-      stk.s2 = push ? s1 : (pop ? s3 : s2);
-      stk.s3 = push ? s2 : s3;
-      stk.count = push ? (stk.count < 4u ? stk.count + 1u : 4u)
-                       : (pop ? (emptied ? 1u : stk.count - 1u) : stk.count);
-      if (LOD) mip_level += push ? -1.0f : (pop ? 1.0f : 0.0f);
-      bounds = next_bounds;
-      target = next_target;
-      // the next iteration would be one too many
-      if (end == RUNS && steps >= t.max_steps) end = GUARD;
     }
-  } while (end == RUNS);
+    // PUSH shifts the stack down (its oldest entry drops out once four are
+    // held), POP shifts it up, and a POP that empties it is followed by the
+    // restart's push of the root; ADVANCE leaves it
+    const uint32_t s0 = stk.s0, s1 = stk.s1, s2 = stk.s2, s3 = stk.s3;
+    stk.s0 = push ? tword : (pop ? (emptied ? 0u : s1) : s0);
+    stk.s1 = push ? s0 : (pop ? s2 : s1);
+    stk.s2 = push ? s1 : (pop ? s3 : s2);
+    stk.s3 = push ? s2 : s3;
+    stk.count = push ? (stk.count < 4u ? stk.count + 1u : 4u)
+                     : (pop ? (emptied ? 1u : stk.count - 1u) : stk.count);
+    if (LOD) w.mip_level += push ? -1.0f : (pop ? 1.0f : 0.0f);
+    bounds = next_bounds;
+    target = next_target;
+    // the next iteration would be one too many
+    if (end == WALK_RUNS && steps >= t.max_steps) end = WALK_GUARD;
+  }
+}
+
+// The result of a ray whose walk has ended.
+template <bool LOD, bool P2>
+SVO_HD __attribute__((always_inline)) inline CastResult walk_result(const TreeView& t,
+                                                                   const NodeRec* top,
+                                                                   uint32_t ntop, RayWalk& w) {
+  CastResult r;
+  r.hit = 0;
+  r.flags = w.flags;
+  uint32_t end = w.end;
 #if defined(__HIP_DEVICE_COMPILE__)
   // (opaque here, so that the tests below are not carried through the loop)
   asm volatile("" : "+v"(end));
 #endif
-  if (end == CRAWL) return crawl_out_of_root(t, p, d, steps, r.flags);
-  if (end == GUARD) r.flags |= FLAG_ITERATION_GUARD;
-  const bool mip = LOD && end == HIT_MIP;
-  if (end == HIT || mip) {
+  if (end == WALK_CRAWL) return crawl_out_of_root(t, w.p, w.d, w.steps, r.flags);
+  if (end == WALK_GUARD) r.flags |= FLAG_ITERATION_GUARD;
+  const bool mip = LOD && end == WALK_HIT_MIP;
+  if (end == WALK_HIT || mip) {
     // the brick that was hit, from the state the hit left as it was
-    const NodeRec& n = (stk.s0 < ntop ? top : t.nodes)[stk.s0];
+    const NodeRec& n = (w.stk.s0 < ntop ? top : t.nodes)[w.stk.s0];
     const uint32_t meta = n.meta;
     const bool uniform = node_kind(meta) == KIND_UNIFORM_LEAF;
     const bool whole = uniform || mip;
-    const uint32_t slot = uniform ? 0u : target & 7u;  // (unused by a MIP hit)
-    const Cube tb = child_bounds_for(bounds, target);
-    const Cube bb{V3f{whole ? bounds.min.x : tb.min.x, whole ? bounds.min.y : tb.min.y,
-                      whole ? bounds.min.z : tb.min.z},
-                  whole ? bounds.size : tb.size};
+    const uint32_t slot = uniform ? 0u : w.target & 7u;  // (unused by a MIP hit)
+    const Cube tb = child_bounds_for(w.bounds, w.target);
+    const Cube bb{V3f{whole ? w.bounds.min.x : tb.min.x, whole ? w.bounds.min.y : tb.min.y,
+                      whole ? w.bounds.min.z : tb.min.z},
+                  whole ? w.bounds.size : tb.size};
     brick_hit<P2>(t, mip ? n.mip : brick_form(meta, slot), mip ? n.mip_word : n.child[slot], bb,
-                  cell, p, &r);
+                  w.cell, w.p, &r);
   }
   return r;
+}
+
+template <bool LOD, bool P2, class LutT>
+SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
+    const TreeView& t, const LutT* __restrict__ lut, V3f o, V3f d, const NodeRec* top,
+    uint32_t ntop, float viewing_distance) {
+  RayWalk w;
+  walk_begin<LOD>(t, o, d, w);
+  if (w.end != WALK_RUNS) return miss_flags(0u);
+  do {
+    walk_iterate<LOD, P2, 0>(t, lut, o, top, ntop, viewing_distance, w);
+  } while (w.end == WALK_RUNS);
+  return walk_result<LOD, P2>(t, top, ntop, w);
 }
 
 // The same traversal as cast_ray_impl<false, P2> with the work of a wave
