@@ -60,15 +60,17 @@ __global__ __launch_bounds__(64) void cast_lod_kernel(TreeView t, const float* _
 // A large ray array, mostly of rays that have little to do with each other:
 // each wave owns `per_wave` consecutive rays and its lanes take them one after
 // another. Neighbouring rays differ in length and in what each iteration does,
-// so a wave of one ray per lane has 7-14% of its lanes active on average. Two
-// things raise that: lanes whose ray has ended take the next rays as soon as
-// kRefill of them wait (results are stored and rays set up for them together),
-// and a lane walks at most kSlice brick cells per iteration, so that the others
-// do not wait for the longest walk of the wave (walk_iterate's slices).
-// (kSlice 2 / 4 / 6 / 8 / 16 on 3M rays: spheres 512^3 - / 873 / 822 / 818 /
-// 921 us, caves 512^3 967 / 877 / 895 / 975 / 1130; kRefill 16 and 32 measured
-// within 3% of 24.)
-constexpr int kSlice = 6;
+// so a wave of one ray per lane has 7-14% of its lanes active on average.
+// Three things raise that: lanes whose ray has ended take the next rays as soon
+// as kRefill of them wait (results are stored and rays set up for them
+// together); a brick walk goes on for at most kSlice cells at a time, so that
+// the others do not wait for the longest; and each pass is either a walk of the
+// lanes that stand in a brick or a stack-loop iteration of the rest, whichever
+// are more. 3M rays into spheres 512^3 and caves 512^3, kSlice 4 / 8 / 12 / 16 /
+// 24: 923 / 836 / 808 / 790 / 772 and 896 / 841 / 824 / 818 / 826 us; both parts
+// in every pass, kSlice 6: 820 and 893 us. (kRefill 16 and 32, and lines at a
+// third and two thirds instead of half, measured within 3%.)
+constexpr int kSlice = 20;
 constexpr uint32_t kRefill = 24;
 template <bool LOD>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6)))
@@ -82,8 +84,9 @@ void cast_stream_kernel(TreeView t, const float* __restrict__ rays, uint32_t n,
   RayWalk w;
   walk_begin<LOD>(t, o, V3f{1.0f, 1.0f, 1.0f}, w);
   w.end = WALK_MISS;
-  // Ends: each pass either iterates a running ray (whose iterations are
-  // bounded), or stores and takes rays, of which there are finitely many.
+  // Ends: each pass either takes a running ray further (whose iterations and
+  // walks are bounded), or stores and takes rays, of which there are finitely
+  // many.
   for (;;) {
     const uint64_t running = __ballot(w.end == WALK_RUNS);
     const uint32_t idle = 64u - static_cast<uint32_t>(__popcll(running));
@@ -110,8 +113,12 @@ void cast_stream_kernel(TreeView t, const float* __restrict__ rays, uint32_t n,
       if (running == 0ull && __ballot(i != kNone) == 0ull) break;
       continue;
     }
-    if (w.end == WALK_RUNS)
-      walk_iterate<LOD, true, kSlice>(t, t.ray_lut, o, nullptr, 0u, viewing_distance, w);
+    const uint64_t due = __ballot(w.end == WALK_RUNS && w.brick == BRICK_DUE);
+    if (2 * __popcll(due) >= __popcll(running)) {
+      if (w.end == WALK_RUNS && w.brick == BRICK_DUE) walk_slice<true, kSlice>(t, nullptr, 0u, w);
+    } else if (w.end == WALK_RUNS && w.brick != BRICK_DUE) {
+      walk_iterate<LOD, true, true>(t, t.ray_lut, o, nullptr, 0u, viewing_distance, w);
+    }
   }
 }
 
@@ -1095,14 +1102,14 @@ uint32_t cast_order_threshold() { return g_cast_order_threshold.load(); }
 
 // More rays than lanes run at once: from there on a lane has further rays to
 // take. 3M rays in their own order, streamed against one ray per lane ordered
-// by origin and direction (order.hip; its sort is 0.2 ms): spheres 512^3 0.82
-// against 1.20 ms, caves 512^3 0.90 against 1.37; 1.2M rays, caves 0.44
+// by origin and direction (order.hip; its sort is 0.2 ms): spheres 512^3 0.78
+// against 1.20 ms, caves 512^3 0.82 against 1.37; 1.2M rays, caves 0.41
 // against 0.69; one ray per lane unordered: 1.42, 1.18 and 0.54 ms. Around the
-// line: 300,007 rays 188 streamed, 152 us one per lane; 500,000 rays 233 and
+// line: 300,007 rays 188 streamed, 152 us one per lane; 500,000 rays 228 and
 // 245 us.
 // LOD rays end sooner and gain less, so for them the line is twice as far:
 // 500,009 rays 196 us streamed, 184 one per lane; 1M rays 291 and 295; 3M into
-// a 256^3 heightfield 715 and 999.
+// a 256^3 heightfield 660 and 999.
 bool streams_cast(uint64_t n, bool lod) {
   const uint32_t order_from = chosen_order_threshold();
   return n > uint64_t(kStreamWaves) * (lod ? 128u : 64u) && (order_from == 0u || n < order_from);

@@ -616,8 +616,10 @@ struct RayWalk {
   uint32_t steps, flags;
   uint32_t cell;     // flat cell of a hit, or of a sliced walk that goes on (else NO_CELL)
   uint32_t end;      // WALK_*
+  uint32_t brick;    // deferred walks: BRICK_*, of the iteration under way
   float mip_level;   // LOD
 };
+enum : uint32_t { BRICK_NONE = 0, BRICK_DUE = 1, BRICK_DONE = 2 };
 enum : uint32_t {
   WALK_RUNS = 0,
   WALK_HIT = 1,
@@ -644,6 +646,7 @@ SVO_HD __attribute__((always_inline)) inline void walk_begin(const TreeView& t, 
   w.steps = 0;
   w.flags = 0;
   w.cell = NO_CELL;
+  w.brick = BRICK_NONE;
   w.end = ir != 0 ? WALK_RUNS : WALK_MISS;
   // log2(size / dim) of two powers of two, exactly
   w.mip_level =
@@ -652,9 +655,10 @@ SVO_HD __attribute__((always_inline)) inline void walk_begin(const TreeView& t, 
 
 // One iteration of the reference's stack loop and, when the stack has
 // emptied, its restart from the root (which ends the ray when the nudged point
-// leaves the tree). With SLICE > 0 a brick walk takes at most SLICE steps in
-// one call, and the calls that carry it on are not iterations.
-template <bool LOD, bool P2, int SLICE, class LutT>
+// leaves the tree). With DEFER an iteration that meets a Parted brick of a
+// leaf only marks it due; walk_slice walks it, and the next call goes on with
+// the iteration from there.
+template <bool LOD, bool P2, bool DEFER, class LutT>
 SVO_HD __attribute__((always_inline)) inline void walk_iterate(
     const TreeView& t, const LutT* __restrict__ lut, V3f o, const NodeRec* top, uint32_t ntop,
     float viewing_distance, RayWalk& w) {
@@ -680,9 +684,8 @@ SVO_HD __attribute__((always_inline)) inline void walk_iterate(
   asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z));
 #endif
   V3f sig{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
-  const bool fresh = SLICE == 0 || w.cell == NO_CELL;
+  const bool fresh = !DEFER || w.brick == BRICK_NONE;
   if (fresh) ++steps;  // (against the bound at the iteration's end)
-  bool more = false;
   const uint32_t key = stk.s0;
   const NodeRec& n = (key < ntop ? top : t.nodes)[key];
   const uint64_t occ = n.occ;
@@ -718,18 +721,21 @@ SVO_HD __attribute__((always_inline)) inline void walk_iterate(
       }
     }
   }
-  if ((!LOD || end == WALK_RUNS) && target != OOB_OCTANT &&
+  if ((!LOD || end == WALK_RUNS) && fresh && target != OOB_OCTANT &&
       (kind == KIND_UNIFORM_LEAF || kind == KIND_LEAF)) {
     const uint32_t slot = uniform ? 0u : target;
     const uint32_t form = brick_form(meta, slot);
     if (form == FORM_SOLID) end = WALK_HIT;
     if (form == FORM_PARTED) {
-      if (walk_brick<P2, SLICE>(t, slot == target ? tword : n.child[0],
-                         uniform ? bounds : child_bounds_for(bounds, target), d, sig, scale,
-                         &p, &w.cell, &w.flags, &more))
-        end = WALK_HIT;
-      if (SLICE > 0 && end == WALK_RUNS && !more) w.cell = NO_CELL;
-      moved_by_probe();
+      if constexpr (DEFER) {
+        w.brick = BRICK_DUE;
+      } else {
+        if (walk_brick<P2>(t, slot == target ? tword : n.child[0],
+                           uniform ? bounds : child_bounds_for(bounds, target), d, sig, scale,
+                           &p, &w.cell, &w.flags))
+          end = WALK_HIT;
+        moved_by_probe();
+      }
     }
   }
   // signum(d) formed again past the probe, so that the values formed
@@ -738,7 +744,8 @@ SVO_HD __attribute__((always_inline)) inline void walk_iterate(
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("" : "+v"(d.x), "+v"(d.y), "+v"(d.z), "+v"(end));
 #endif
-  if ((SLICE == 0 || !more) && end == WALK_RUNS) {
+  if ((!DEFER || w.brick != BRICK_DUE) && end == WALK_RUNS) {
+    if constexpr (DEFER) w.brick = BRICK_NONE;
     sig = V3f{sign_one(d.x), sign_one(d.y), sign_one(d.z)};
     // (an empty bitmap has nothing ahead)
     const bool pop = uniform | (target == OOB_OCTANT) | ((occ & ahead) == 0ull);
@@ -848,6 +855,30 @@ SVO_HD __attribute__((always_inline)) inline void walk_iterate(
   }
 }
 
+// At most SLICE steps through the brick that walk_iterate marked due.
+template <bool P2, int SLICE>
+SVO_HD __attribute__((always_inline)) inline void walk_slice(const TreeView& t, const NodeRec* top,
+                                                            uint32_t ntop, RayWalk& w) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(w.d.x), "+v"(w.d.y), "+v"(w.d.z));
+#endif
+  const V3f sig{sign_one(w.d.x), sign_one(w.d.y), sign_one(w.d.z)};
+  const NodeRec& n = (w.stk.s0 < ntop ? top : t.nodes)[w.stk.s0];
+  const bool uniform = node_kind(n.meta) == KIND_UNIFORM_LEAF;
+  const Cube tb = child_bounds_for(w.bounds, w.target);
+  const Cube bb{V3f{uniform ? w.bounds.min.x : tb.min.x, uniform ? w.bounds.min.y : tb.min.y,
+                    uniform ? w.bounds.min.z : tb.min.z},
+                uniform ? w.bounds.size : tb.size};
+  bool more = false;
+  if (walk_brick<P2, SLICE>(t, n.child[uniform ? 0u : w.target & 7u], bb, w.d, sig, w.scale, &w.p,
+                            &w.cell, &w.flags, &more)) {
+    w.end = WALK_HIT;
+  } else if (!more) {
+    w.cell = NO_CELL;
+    w.brick = BRICK_DONE;
+  }
+}
+
 // The result of a ray whose walk has ended.
 template <bool LOD, bool P2>
 SVO_HD __attribute__((always_inline)) inline CastResult walk_result(const TreeView& t,
@@ -889,7 +920,7 @@ SVO_HD __attribute__((always_inline)) inline CastResult cast_ray_impl(
   walk_begin<LOD>(t, o, d, w);
   if (w.end != WALK_RUNS) return miss_flags(0u);
   do {
-    walk_iterate<LOD, P2, 0>(t, lut, o, top, ntop, viewing_distance, w);
+    walk_iterate<LOD, P2, false>(t, lut, o, top, ntop, viewing_distance, w);
   } while (w.end == WALK_RUNS);
   return walk_result<LOD, P2>(t, top, ntop, w);
 }
