@@ -633,14 +633,13 @@ template <bool LOD>
 SVO_HD __attribute__((always_inline)) inline void walk_begin(const TreeView& t, V3f o, V3f d,
                                                             RayWalk& w) {
   w.d = d;
-  w.scale = dda_scale_factors(d);
   w.dir_idx = hash_direction(d);
   // (for a NaN component every scale factor is NaN and no step moves any axis)
   w.neg = octant_of(__builtin_signbit(d.x), __builtin_signbit(d.y), __builtin_signbit(d.z));
   w.bounds = Cube{v3u(0.0f), t.size};
   w.stk = RingStack{0u, 0u, 0u, 0u, 1u};  // the root pushed
   float tt = 0.0f;
-  const int ir = intersect_ray(w.bounds, o, d, &tt);
+  const int ir = ray_setup(w.bounds, o, d, &tt, &w.scale);
   w.p = ir != 0 ? o + d * (ir == 2 ? tt : 0.0f) : o;
   w.target = hash_region(w.p - w.bounds.min, w.bounds.size / 2.0f);
   w.steps = 0;
