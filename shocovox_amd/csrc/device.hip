@@ -1105,7 +1105,7 @@ uint32_t cast_order_threshold() { return g_cast_order_threshold.load(); }
 // by origin and direction (order.hip; its sort is 0.2 ms): spheres 512^3 0.78
 // against 1.20 ms, caves 512^3 0.82 against 1.37; 1.2M rays, caves 0.41
 // against 0.69; one ray per lane unordered: 1.42, 1.18 and 0.54 ms. Around the
-// line: 300,007 rays 188 streamed, 152 us one per lane; 500,000 rays 228 and
+// line: 300,007 rays 188 streamed, 152 us one per lane; 500,000 rays 214 and
 // 245 us.
 // LOD rays end sooner and gain less, so for them the line is twice as far:
 // 500,009 rays 196 us streamed, 184 one per lane; 1M rays 291 and 295; 3M into
@@ -1118,7 +1118,9 @@ bool streams_cast(uint64_t n, bool lod) {
 int launch_cast_stream(const DeviceTree& t, const float* rays, uint32_t n, float viewing_distance,
                        bool lod, const svo_hits& out, void* stream, std::string* err) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const uint32_t per = (n - 1u) / kStreamWaves + 1u;
+  // (at least two rays a lane, with fewer waves instead: 500,000 rays 226 us
+  // with 82 a wave, 214 with 128)
+  const uint32_t per = std::max((n - 1u) / kStreamWaves + 1u, 128u);
   const dim3 grid((n - 1u) / per + 1u);
   if (lod)
     hipLaunchKernelGGL(cast_stream_kernel<true>, grid, dim3(64), 0, s, t.view, rays, n,
