@@ -606,6 +606,13 @@ struct RingStack {
 // Together a lone ray's iteration takes 0.56 us instead of 0.78, 8 1080p
 // frames in one batched run 0.90 ms instead of 0.96, one of them 0.185 ms
 // instead of 0.208.
+// lut[i] by a 32-bit byte offset, which the load adds to the base itself (a
+// 64-bit index is added by the vector unit first: 1080p frame 165 -> 163 us,
+// 4K 499 -> 492).
+template <class LutT>
+SVO_HD inline uint64_t lut_word(const LutT* lut, uint32_t i) {
+  return *reinterpret_cast<const LutT*>(reinterpret_cast<const char*>(lut) + (i << 3));
+}
 struct RayWalk {
   V3f d, scale, p;
   Cube bounds;
@@ -698,10 +705,10 @@ SVO_HD __attribute__((always_inline)) inline void walk_iterate(
   // continues from it, the cell index comes from bitmap_cell
   const float rcp_size = size_rcp<P2>(bounds.size);
   V3f bp = bitmap_pos<P2>(p, bounds, rcp_size);
-  uint64_t ahead = lut[bitmap_cell(bp) * 8u + dir_idx];
+  uint64_t ahead = lut_word(lut, bitmap_cell(bp) * 8u + dir_idx);
   auto moved_by_probe = [&]() {
     bp = bitmap_pos<P2>(p, bounds, rcp_size);
-    ahead = lut[bitmap_cell(bp) * 8u + dir_idx];
+    ahead = lut_word(lut, bitmap_cell(bp) * 8u + dir_idx);
 #if defined(__HIP_DEVICE_COMPILE__)
     // (used here, so that the two requests are not merged into one after
     // the probe)
@@ -816,7 +823,7 @@ SVO_HD __attribute__((always_inline)) inline void walk_iterate(
           bp = bp + move;
           // stop at a reachable occupied child or a non-empty leaf brick;
           // both words are requested together, whichever the test needs
-          const uint64_t there = lut[bitmap_index(bp, &w.flags) * 8u + dir_idx];
+          const uint64_t there = lut_word(lut, bitmap_index(bp, &w.flags) * 8u + dir_idx);
           const uint32_t word = n.child[next_target];
           const bool child = (kind == KIND_INTERNAL) &
                              ((occ & octant_bitmap_mask(next_target)) != 0ull) &
