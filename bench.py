@@ -38,11 +38,12 @@ sys.path.insert(0, str(ROOT))
 
 METRIC = ("Mrays/s at 1080p into 512³; p50/p99 latency batched vs per-call at fixed QPS")
 HBM_PEAK_GBS = 8000.0
-# VALU issue ceiling of an MI355X in G wave64 instructions per second: each
-# of a CU's 4 SIMDs is 16 lanes wide and issues one wave64 VALU instruction
-# every 4 cycles, so a CU completes one per cycle; 256 CUs at the 2.4 GHz
-# peak engine clock.
-VALU_PEAK_GIPS = 256 * 1.0 * 2.4
+# VALU issue ceiling of an MI355X in G wave64 instructions per second: the
+# part's FP32 vector rate is 256 flops per CU and cycle, which is two wave64
+# multiply-adds; 256 CUs at the 2.4 GHz peak engine clock. (One instruction per
+# SIMD every four cycles, half of that, is exceeded by these kernels: 0.29 per
+# SIMD and cycle measured.)
+VALU_PEAK_GIPS = 256 * 2.0 * 2.4
 # Algorithmic bytes of one logical event of the reference traversal
 EVENT_BYTES = {"stack_iterations": 12, "child_reads": 4, "brick_reads": 4, "voxel_tests": 8,
                "data_palette_reads": 4, "hits": 4}
@@ -202,10 +203,10 @@ def batched_bench(args, render_variant: str) -> dict:
             dtrees[ti].render_into(vp, w, h, b, stream)
 
     # the per-viewport baseline runs the render variant fastest on this pool,
-    # among the headline's pick and the two forms of the one-tile kernel
+    # among the headline's pick, the frame kernel and two forms of the one-tile kernel
     rnames = render_variants()
     cands = []
-    for name in (render_variant, "w5-glut-8x8", "w5-glut-8x8-ww-g1"):
+    for name in (render_variant, "auto", "w5-glut-8x8", "w5-glut-8x8-ww-g1"):
         if name in rnames and name not in cands:
             cands.append(name)
     plain_ms = {}
@@ -542,7 +543,8 @@ def spheres_block(args) -> dict:
     ref = [{k: b[k].clone() for k in fields} for b in (pr, pc)]
     names = batch_variants()
     tuning = {}
-    for name in ("classic-w5-g5", "classic-w6-g6", "ww-w5-g5", "ww-w6-g6", "classic-w5-g5-n73"):
+    for name in ("auto", "classic-w5-g5", "classic-w6-g6", "ww-w5-g5", "ww-w6-g6",
+                 "classic-w5-g5-n73"):
         if name not in names:
             continue
         select_batch_variant(names.index(name))
