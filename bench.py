@@ -794,10 +794,12 @@ def main() -> int:
         # per-frame render launch (the render rays of one pose)
         if batch is not None:
             rays_per_launch, launch_ms, kname = rays_per_step, avg_launch_ms, "batch_kernel"
+            picked = bvariant
         else:
             rays_per_launch = rays_per_frame
             launch_ms = tuning.get(best) if tuning else pf_ms / len(vps)
             kname = "render_kernel"
+            picked = best
         achieved = b_ray * rays_per_launch / (launch_ms * 1e-3) / 1e9
         traffic = None
         counters = {}
@@ -809,7 +811,9 @@ def main() -> int:
         tf = ROOT / "profiles" / f"{kname}_{cfg.name}_{cfg.height}p_traffic.json"
         if tf.exists():
             tj = json.loads(tf.read_text())
-            if tj.get("units_per_launch") == rays_per_launch:
+            # (counters of one kernel say nothing about another variant)
+            if tj.get("units_per_launch") == rays_per_launch and tj.get("variant") == picked:
+                kname = tj["kernel"]
                 traffic = tj.get("bytes_per_launch")
                 counters = {k: tj[k] for k in ("l2_hit_rate", "valu_lane_utilization")
                             if k in tj}
