@@ -399,7 +399,9 @@ __global__ __launch_bounds__(256) void upload_table_kernel(uint32_t* __restrict_
 }
 
 // Writes `bytes` of a table (a multiple of 4) to the device by upload kernels.
-void upload_table(void* dst, const char* src, size_t bytes, hipStream_t s) {
+// (Launch errors are returned by whoever asks for them first, so each helper
+// returns its own, and no kernel is launched on a table that did not arrive.)
+hipError_t upload_table(void* dst, const char* src, size_t bytes, hipStream_t s) {
   const uint32_t words = static_cast<uint32_t>((bytes + 3) / 4);
   for (uint32_t w0 = 0; w0 < words; w0 += kUploadWords) {
     UploadChunk c;
@@ -408,7 +410,10 @@ void upload_table(void* dst, const char* src, size_t bytes, hipStream_t s) {
     std::memcpy(c.words, src + static_cast<size_t>(w0) * 4, static_cast<size_t>(c.count) * 4);
     hipLaunchKernelGGL(upload_table_kernel, dim3(1), dim3(256), 0, s,
                        static_cast<uint32_t*>(dst), c);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
+  return hipSuccess;
 }
 
 // Tables up to this size go by upload kernels (four of them), larger ones by a
@@ -787,7 +792,7 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
   if (b->pending[slot ^ 1u]) e = hipStreamWaitEvent(s, b->done[slot ^ 1u], 0);
   if (per_tile) {
     if (e == hipSuccess && used <= kUploadBytes)
-      upload_table(b->dev, base, used, s);
+      e = upload_table(b->dev, base, used, s);
     else if (e == hipSuccess)
       e = hipMemcpyAsync(b->dev, base, used, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = launch_tiles(static_cast<const char*>(b->dev), n, tiles, any_lod, s);
@@ -943,18 +948,18 @@ int run_static(const svo_job* jobs, uint32_t n, void* stream, std::string* err) 
   fill_header(base, n, tiles, trees_offset);
   const size_t used = trees_offset + ntrees * sizeof(TreeView);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  upload_table(sd->scratch, base, used, s);
-  if (v.per_tile) {
-    (void)launch_tiles(sd->scratch, n, tiles, any_lod, s);
-  } else {
+  e = upload_table(sd->scratch, base, used, s);
+  if (e == hipSuccess && v.per_tile) {
+    e = launch_tiles(sd->scratch, n, tiles, any_lod, s);
+  } else if (e == hipSuccess) {
     Counter* counters = reinterpret_cast<Counter*>(sd->scratch + kStaticCountersOffset);
     hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, s, counters);
     const BatchFn fn = any_lod ? v.lod_fn : v.fn;
     const uint32_t grid = sd->cus * v.groups_per_cu;
     hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, s, static_cast<const char*>(sd->scratch),
                        counters);
+    e = hipGetLastError();
   }
-  e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "svo_batch_run_static launch", err);
   return SVO_OK;
 }

@@ -1,0 +1,50 @@
+"""What batched runs answer when a launch fails, and what they keep of the work
+queued before it: on the CPU, with a stand-in for the HIP runtime that logs
+every call and fails the launches it is told to."""
+from __future__ import annotations
+
+import pytest
+
+import fakehip
+
+PRELUDE = """
+import sys
+sys.modules["torch"] = None  # (its libraries would register their kernels with the stand-in)
+import ctypes as C
+import numpy as np
+from shocovox_amd import DeviceTree, Octree, _native as N, workloads as W
+L = N.lib()
+F = C.CDLL({lib!r})
+F.fake_log.restype = C.c_char_p
+F.fake_news.restype = C.c_ulong
+tree = DeviceTree(Octree.scene(2, 64, 4, 3))
+vp = W.look_at_viewport((90.0, 80.0, -20.0), (32.0, 30.0, 32.0), 40, 24)
+rays = np.zeros((400_000, 6), np.float32)  # (never read here)
+def render():
+    return N.Job(tree._h, 0, 40, 24, vp.to_c(), None, N.Hits(), 0.0)
+def cast(n):
+    return N.Job(tree._h, 1, n, 1, N.Viewport(), rays.ctypes.data, N.Hits(), 0.0)
+def jobs(*js):
+    return (N.Job * len(js))(*js)
+def log():
+    return [l.split() for l in F.fake_log().decode().splitlines()]
+def error():
+    return L.svo_last_error().decode()
+S = [C.c_void_p(0x1000), C.c_void_p(0x2000)]  # (streams the stand-in only logs)
+""".format(lib=str(fakehip.LIB))
+
+
+@pytest.mark.parametrize("kernel", ["upload_table_kernel", "batch_tile_kernel"])
+def test_static_run_reports_a_failed_launch(kernel):
+    fakehip.run(PRELUDE + f"""
+js = jobs(render())
+assert L.svo_batch_run_static(js, 1, S[0]) == 0
+F.fake_clear_log()
+F.fake_fail_launch({kernel!r}.encode())
+assert L.svo_batch_run_static(js, 1, S[0]) == 7, log()
+assert "launch" in error(), error()
+# nothing runs on a table that did not arrive
+assert not any(l[0] == "launch" and "batch_tile" in l[1] for l in log()), log()
+F.fake_fail_launch(b"")
+assert L.svo_batch_run_static(js, 1, S[0]) == 0
+""")
