@@ -516,21 +516,20 @@ hipError_t launch_tiles(const char* table, uint32_t n, uint64_t tiles, bool lod,
   return hipGetLastError();
 }
 
-// Job i of a per-tile run: like fill_job, but a large ray array keeps no tiles
-// and is listed in `streamed`, to run by its own launch (launch_cast_stream).
-// *all counts the tiles of both kinds.
-int fill_job_or_stream(BatchJob& j, const BatchJobIn& in, uint32_t i, uint32_t ti, bool per_tile,
-                       uint32_t tw, uint32_t th, uint64_t* tiles, uint64_t* all, bool* lod,
-                       std::vector<uint32_t>* streamed, std::string* err) {
-  const bool stream = per_tile && in.kind == 1 && in.rays &&
-                      streams_cast(in.width, in.viewing_distance > 0.0f);
+// A job of a per-tile run: like fill_job, but a large ray array keeps no tiles
+// and sets *stream, to run by its own launch (launch_cast_stream). *all counts
+// the tiles of both kinds.
+int fill_job_or_stream(BatchJob& j, const BatchJobIn& in, uint32_t ti, bool per_tile, uint32_t tw,
+                       uint32_t th, uint64_t* tiles, uint64_t* all, bool* lod, bool* stream,
+                       std::string* err) {
+  *stream = per_tile && in.kind == 1 && in.rays &&
+            streams_cast(in.width, in.viewing_distance > 0.0f);
   bool job_lod = false;
   const int st = fill_job(j, in, ti, tw, th, all, &job_lod, err);
   if (st != SVO_OK) return st;
   j.tile_begin = static_cast<uint32_t>(*tiles);
-  if (stream) {
+  if (*stream) {
     j.tile_count = 0;
-    streamed->push_back(i);
   } else {
     *tiles += j.tile_count;
     *lod = *lod || job_lod;
@@ -751,9 +750,11 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
     } else {
       ti = it->second;
     }
-    const int st = fill_job_or_stream(out[i], in, i, ti, v.per_tile, v.tile_w, v.tile_h, &tiles,
-                                      &all_tiles, &any_lod, &streamed, err);
+    bool stream = false;
+    const int st = fill_job_or_stream(out[i], in, ti, v.per_tile, v.tile_w, v.tile_h, &tiles,
+                                      &all_tiles, &any_lod, &stream, err);
     if (st != SVO_OK) return st;
+    if (stream) streamed.push_back(i);
   }
   // large cast jobs traverse their rays in svo_cast's order (kernels on `s`
   // ahead of the graph; the orders go back to the pool after it)
@@ -902,7 +903,7 @@ int run_static(const svo_job* jobs, uint32_t n, void* stream, std::string* err) 
   const BatchVariant& v = kBatchVariants[g_batch_variant];
   uint64_t tiles = 0, all_tiles = 0;
   bool any_lod = false;
-  std::vector<uint32_t> streamed;
+  uint32_t streamed[kStaticMaxJobs], nstreamed = 0;
   for (uint32_t i = 0; i < n; ++i) {
     const svo_job& j = jobs[i];
     if (!j.tree || !j.tree->dev || j.tree->dev->device != device) {
@@ -934,12 +935,14 @@ int run_static(const svo_job* jobs, uint32_t n, void* stream, std::string* err) 
       keys[ntrees++] = in.tree;
       trees[ti] = in.tree->view;
     }
-    st = fill_job_or_stream(out[i], in, i, ti, v.per_tile, v.tile_w, v.tile_h, &tiles, &all_tiles,
-                            &any_lod, &streamed, err);
+    bool stream = false;
+    st = fill_job_or_stream(out[i], in, ti, v.per_tile, v.tile_w, v.tile_h, &tiles, &all_tiles,
+                            &any_lod, &stream, err);
     if (st != SVO_OK) return st;
+    if (stream) streamed[nstreamed++] = i;
   }
-  for (uint32_t i : streamed) {
-    const svo_job& j = jobs[i];
+  for (uint32_t k = 0; k < nstreamed; ++k) {
+    const svo_job& j = jobs[streamed[k]];
     st = launch_cast_stream(*j.tree->dev, j.rays, j.width, j.viewing_distance,
                             j.viewing_distance > 0.0f, j.out, stream, err);
     if (st != SVO_OK) return st;

@@ -48,3 +48,16 @@ assert not any(l[0] == "launch" and "batch_tile" in l[1] for l in log()), log()
 F.fake_fail_launch(b"")
 assert L.svo_batch_run_static(js, 1, S[0]) == 0
 """)
+
+
+def test_static_run_allocates_nothing():
+    """svo_batch_run_static makes no allocation on the host either, so it
+    cannot run out of memory between two of its launches."""
+    fakehip.run(PRELUDE + """
+js = jobs(cast(400_000), render(), cast(400_000), cast(100))
+for _ in range(2):
+    before = F.fake_news()
+    assert L.svo_batch_run_static(js, 4, S[0]) == 0
+    after = F.fake_news()
+assert after == before, (before, after)
+""")
