@@ -790,6 +790,7 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
     }
   }
   hipError_t e = hipSuccess;
+  int st = SVO_OK;
   if (b->pending[slot ^ 1u]) e = hipStreamWaitEvent(s, b->done[slot ^ 1u], 0);
   if (per_tile) {
     if (e == hipSuccess && used <= kUploadBytes)
@@ -797,15 +798,10 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
     else if (e == hipSuccess)
       e = hipMemcpyAsync(b->dev, base, used, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = launch_tiles(static_cast<const char*>(b->dev), n, tiles, any_lod, s);
-    int st = SVO_OK;
     for (size_t k = 0; k < streamed.size() && e == hipSuccess && st == SVO_OK; ++k) {
       const BatchJobIn& in = jobs[streamed[k]];
       st = launch_cast_stream(*in.tree, in.rays, in.width, in.viewing_distance,
                               in.viewing_distance > 0.0f, in.out, s, err);
-    }
-    if (st != SVO_OK) {
-      for (uint32_t* p : orders) (void)hipFreeAsync(p, s);
-      return st;
     }
   } else {
     hipGraphExec_t exec = any_lod ? b->exec_lod : b->exec;
@@ -815,12 +811,18 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
     if (e == hipSuccess) e = hipGraphLaunch(exec, s);
   }
   for (uint32_t* p : orders) (void)hipFreeAsync(p, s);
-  if (e != hipSuccess) return hip_fail(e, "batch launch", err);
+  if (e != hipSuccess) st = hip_fail(e, "batch launch", err);
+  // A run that failed on the way may have queued its table's copy and some of
+  // its launches: the next runs have to wait for them all the same.
   e = hipEventRecord(b->done[slot], s);
-  if (e != hipSuccess) return hip_fail(e, "hipEventRecord", err);
-  b->pending[slot] = true;
-  b->next = slot ^ 1u;
-  return SVO_OK;
+  if (e == hipSuccess) {
+    b->pending[slot] = true;
+    b->next = slot ^ 1u;
+  } else {
+    (void)hipStreamSynchronize(s);  // nothing to wait for them by
+    if (st == SVO_OK) st = hip_fail(e, "hipEventRecord", err);
+  }
+  return st;
 }
 
 // ---------------------------------------------------------------------------

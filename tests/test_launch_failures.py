@@ -61,3 +61,46 @@ for _ in range(2):
     after = F.fake_news()
 assert after == before, (before, after)
 """)
+
+
+@pytest.mark.parametrize("small", [True, False], ids=["table-by-kernel", "table-by-copy"])
+@pytest.mark.parametrize("kernel,queued", [("cast_stream_kernel", "batch_tile"),
+                                           ("batch_tile_kernel", "table")])
+def test_failed_run_keeps_the_work_it_queued(small, kernel, queued):
+    """A run whose later launch fails has its table (and tiles) queued: the
+    next run, on another stream, waits for them before it writes the device
+    table, fills the other staging, and the one after that waits for this one."""
+    fakehip.run(PRELUDE + f"""
+small, kernel, queued = {small!r}, {kernel!r}, {queued!r}
+b = C.c_void_p()
+assert L.svo_batch_create(64, C.byref(b)) == 0
+js = jobs(cast(400_000), *[render() for _ in range(1 if small else 60)])
+def run(s):
+    F.fake_clear_log()
+    return L.svo_batch_run(b, js, len(js), s)
+F.fake_fail_launch(kernel.encode())
+assert run(S[0]) == 7, log()
+F.fake_fail_launch(b"")
+first = log()
+table = [i for i, l in enumerate(first)
+         if l[0] == "copy" or (l[0] == "launch" and "upload_table" in l[1])]
+assert table and (first[table[0]][0] == "launch") == small, first
+if queued == "batch_tile":
+    assert any(l[0] == "launch" and queued in l[1] for l in first), first
+records = [i for i, l in enumerate(first) if l[0] == "record" and l[2] == "0x1000"]
+assert records and records[-1] > max(i for i, l in enumerate(first) if l[0] != "record"), first
+event = first[records[-1]][1]
+assert run(S[1]) == 0
+second = log()
+waits = [i for i, l in enumerate(second) if l == ["wait", event, "0x2000"]]
+writes = [i for i, l in enumerate(second)
+          if l[0] == "copy" or (l[0] == "launch" and "upload_table" in l[1])]
+assert waits and writes and waits[0] < writes[0], second
+if not small:
+    assert second[writes[0]][2] != first[table[0]][2], (first, second)
+assert run(S[1]) == 0
+assert log()[0] == ["sync", event], log()
+F.fake_clear_log()
+L.svo_batch_destroy(b)
+assert sum(l[0] == "sync" for l in log()) == 2, log()
+""")
