@@ -312,8 +312,9 @@ int svo_cast(const svo_tree* dtree, const float* rays, uint32_t n, const svo_hit
  * svo_cast, svo_cast_at_lod and svo_batch_run's cast jobs traverse the rays in the
  * order of (origin cell on a 64^3 grid of the tree, Morton order; direction
  * octant), found by a radix sort on the call's stream, instead of streaming
- * them. At the default, 2^20, only the persistent batched variants do;
- * 0 never orders; above 2^31 - 1 rays stay unordered. Process-wide.
+ * them; 0 never orders, and above 2^31 - 1 rays stay unordered. Until it is
+ * called, only the persistent batched variants order (from 2^20 rays).
+ * Process-wide.
  * The sort's scratch comes from the device's default memory pool, which is
  * set to keep freed memory for reuse; without device memory for the sort the
  * rays keep their own order. svo_batch_run_static never orders. */

@@ -1083,14 +1083,15 @@ void device_tree_destroy(DeviceTree* t) {
 }
 
 namespace {
-// Ray count from which casts are ordered (set_cast_order_threshold). Left at
-// the default, plain and per-tile launches stream large casts instead.
-constexpr uint32_t kDefaultOrderThreshold = 1u << 20;
-std::atomic<uint32_t> g_cast_order_threshold{kDefaultOrderThreshold};
+// Ray count from which casts are ordered (set_cast_order_threshold). Until a
+// caller has chosen one, plain and per-tile launches stream large casts
+// instead, and the persistent batched variants order from 2^20 rays.
+constexpr uint64_t kNotChosen = ~0ull;
+std::atomic<uint64_t> g_cast_order_threshold{kNotChosen};
 // The threshold where a caller chose one, else 0.
 uint32_t chosen_order_threshold() {
-  const uint32_t n = g_cast_order_threshold.load();
-  return n == kDefaultOrderThreshold ? 0u : n;
+  const uint64_t n = g_cast_order_threshold.load();
+  return n == kNotChosen ? 0u : static_cast<uint32_t>(n);
 }
 
 // Waves of a streamed cast: as many as run at once at six waves per SIMD.
@@ -1098,7 +1099,10 @@ constexpr uint32_t kStreamWaves = 6 * 1024;
 }  // namespace
 
 void set_cast_order_threshold(uint32_t n) { g_cast_order_threshold.store(n); }
-uint32_t cast_order_threshold() { return g_cast_order_threshold.load(); }
+uint32_t cast_order_threshold() {
+  const uint64_t n = g_cast_order_threshold.load();
+  return n == kNotChosen ? 1u << 20 : static_cast<uint32_t>(n);
+}
 
 // More rays than lanes run at once: from there on a lane has further rays to
 // take. 3M rays in their own order, streamed against one ray per lane ordered

@@ -731,8 +731,8 @@ def set_timing(enabled: bool) -> None:
 
 def set_cast_order_threshold(n: int) -> None:
     """svo_cast orders its rays (origin cell, direction octant) from n rays up
-    instead of streaming them (0 never; at the default, 2^20, only the
-    persistent batched variants do). Process-wide."""
+    instead of streaming them (0 never; until it is called, only the persistent
+    batched variants do, from 2^20). Process-wide."""
     _check(N.lib().svo_cast_set_order_threshold(int(n)))
 
 

@@ -149,6 +149,13 @@ hipError_t hipFree(void* p) {
   std::free(p);
   return hipSuccess;
 }
+// No memory pool: ray ordering finds no memory, and says so in the log.
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t*, int) { return hipErrorNotSupported; }
+hipError_t hipMallocAsync(void**, size_t n, hipStream_t s) {
+  note("nopool %zu %p\n", n, static_cast<void*>(s));
+  return hipErrorOutOfMemory;
+}
+hipError_t hipFreeAsync(void*, hipStream_t) { return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
 hipError_t hipHostFree(void* p) { return hipFree(p); }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
