@@ -57,27 +57,55 @@ __global__ __launch_bounds__(64) void cast_lod_kernel(TreeView t, const float* _
   store_result(t, out, i, res, o);
 }
 
-// A large ray array, mostly of rays that have little to do with each other:
-// each wave owns `per_wave` consecutive rays and its lanes take them one after
-// another. Neighbouring rays differ in length and in what each iteration does,
-// so a wave of one ray per lane has 7-14% of its lanes active on average.
-// Three things raise that: lanes whose ray has ended take the next rays as soon
+// A large ray array: the grid's waves all run at once, and each takes the groups
+// of 64 consecutive rays that lie a grid apart (b, b + grid, ..), its lanes one
+// ray after another. Where neighbouring rays have little to do with each other
+// they differ in length and in what each iteration does, so a wave of one ray
+// per lane has 7-14% of its lanes active on average. Three things raise that: lanes whose ray has ended take the next rays as soon
 // as kRefill of them wait (results are stored and rays set up for them
 // together); a brick walk goes on for at most kSlice cells at a time, so that
 // the others do not wait for the longest; and each pass is either a walk of the
 // lanes that stand in a brick or a stack-loop iteration of the rest, whichever
 // are more. 3M rays into spheres 512^3 and caves 512^3, kSlice 4 / 8 / 12 / 16 /
 // 24: 923 / 836 / 808 / 790 / 772 and 896 / 841 / 824 / 818 / 826 us; both parts
-// in every pass, kSlice 6: 820 and 893 us. (kRefill 16 and 32, and lines at a
-// third and two thirds instead of half, measured within 3%.)
+// in every pass, kSlice 6: 820 and 893 us. (20 as 16 and 24; kRefill 16 and 32,
+// and lines at a third and two thirds instead of half, measured within 3%.)
+// Groups a grid apart, because neighbouring rays of a camera's array cost alike:
+// with n / grid consecutive rays a wave the launch lasted as long as the waves
+// that had the horizon. 3840x2160 camera rays in rows of pixels / in 8x8 tiles,
+// caves 512^3: 1351 / 1902 us so, 878 / 624 now (one ray per lane sorted by
+// order.hip: 1186 / 909); heights 1024^3: 3151 / 6202, 1219 / 931 (3400 / 2842);
+// 1280x720 in tiles, caves 512^3: 429, 254 (282). Random rays do not mind: 3M into
+// spheres 512^3 730 and 697 us, 500,000 into caves 256^3 226 and 227.
+// Rays that do belong together (kNear of each other in direction and, over the
+// tree's size, in origin: 8x8 pixels of 720p, not 64 in a row) end together, and
+// mixed with the next group's they would only part; after such a group the lanes
+// wait for all 64: 4K in tiles 748 -> 616 us, 720p in tiles 305 -> 254, random
+// rays unchanged. (In rows kNear of 2^-5 measured the same within 15% either way.)
+// The LOD form needs more than the 80 registers that six waves leave it: 24 bytes
+// of scratch a lane.
 constexpr int kSlice = 20;
 constexpr uint32_t kRefill = 24;
+constexpr float kNear = 0x1p-6f;
+// Whether every component of v is within `by` of the first active lane's (false
+// for a NaN).
+__device__ inline bool near_first(V3f v, float by) {
+  auto off = [](float x) {
+    return fabsf(x - __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))));
+  };
+  return (off(v.x) <= by) & (off(v.y) <= by) & (off(v.z) <= by);
+}
+
 template <bool LOD>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6)))
 void cast_stream_kernel(TreeView t, const float* __restrict__ rays, uint32_t n,
-                        float viewing_distance, uint32_t per_wave, HitPtrs out) {
-  uint64_t next = static_cast<uint64_t>(blockIdx.x) * per_wave;  // of the rays not yet taken
-  const uint64_t last = min(static_cast<uint64_t>(n), next + per_wave);
+                        float viewing_distance, HitPtrs out) {
+  // The wave's rays are numbered 0 .. last - 1: number q is ray q % 64 of its
+  // (q / 64)-th group. (n > 0 and no more waves than groups.)
+  const uint32_t groups = (n - 1u) / 64u + 1u;
+  const uint32_t last = ((groups - 1u - blockIdx.x) / gridDim.x + 1u) * 64u;
+  uint32_t next = 0u;  // the first not yet taken
+  uint32_t refill = kRefill;
   constexpr uint32_t kNone = 0xFFFFFFFFu;
   uint32_t i = kNone;  // this lane's ray
   V3f o{0.0f, 0.0f, 0.0f};
@@ -90,25 +118,32 @@ void cast_stream_kernel(TreeView t, const float* __restrict__ rays, uint32_t n,
   for (;;) {
     const uint64_t running = __ballot(w.end == WALK_RUNS);
     const uint32_t idle = 64u - static_cast<uint32_t>(__popcll(running));
-    if (running == 0ull || (idle >= kRefill && next < last)) {
+    if (running == 0ull || (idle >= refill && next < last)) {
+      bool apart = false;
       if (w.end != WALK_RUNS) {
         if (i != kNone) {
           const CastResult res = walk_result<LOD, true>(t, nullptr, 0u, w);
           const float* r = rays + 6ull * i;
           store_result(t, out, i, res, V3f{r[0], r[1], r[2]});
         }
-        const uint64_t k =
+        const uint32_t q =
             next + __builtin_amdgcn_mbcnt_hi(
                        static_cast<uint32_t>(~running >> 32),
                        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(~running), 0u));
         i = kNone;
-        if (k < last) {
+        // (64 bits: the last group may reach beyond 2^32)
+        const uint64_t k =
+            (static_cast<uint64_t>(q >> 6) * gridDim.x + blockIdx.x) * 64u + (q & 63u);
+        if (q < last && k < n) {
           i = static_cast<uint32_t>(k);
           const float* r = rays + 6ull * i;
           o = V3f{r[0], r[1], r[2]};
-          walk_begin<LOD>(t, o, V3f{r[3], r[4], r[5]}, w);
+          const V3f d{r[3], r[4], r[5]};
+          walk_begin<LOD>(t, o, d, w);
+          apart = !(near_first(d, kNear) & near_first(o, t.size * kNear));
         }
       }
+      refill = running != 0ull || __ballot(apart) != 0ull ? kRefill : 64u;
       next += idle;
       if (running == 0ull && __ballot(i != kNone) == 0ull) break;
       continue;
@@ -1124,14 +1159,14 @@ int launch_cast_stream(const DeviceTree& t, const float* rays, uint32_t n, float
   hipStream_t s = static_cast<hipStream_t>(stream);
   // (at least two rays a lane, with fewer waves instead: 500,000 rays 226 us
   // with 82 a wave, 214 with 128)
-  const uint32_t per = std::max((n - 1u) / kStreamWaves + 1u, 128u);
-  const dim3 grid((n - 1u) / per + 1u);
+  const uint32_t groups = (n - 1u) / 64u + 1u;
+  const dim3 grid(std::min(kStreamWaves, (groups + 1u) / 2u));
   if (lod)
     hipLaunchKernelGGL(cast_stream_kernel<true>, grid, dim3(64), 0, s, t.view, rays, n,
-                       viewing_distance, per, to_ptrs(out));
+                       viewing_distance, to_ptrs(out));
   else
     hipLaunchKernelGGL(cast_stream_kernel<false>, grid, dim3(64), 0, s, t.view, rays, n,
-                       viewing_distance, per, to_ptrs(out));
+                       viewing_distance, to_ptrs(out));
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? SVO_OK : hip_fail(e, "cast_stream_kernel launch", err);
 }
