@@ -189,6 +189,27 @@ __device__ __attribute__((always_inline)) inline void cast_tile(const BatchJob& 
   store_result(tv, held_ptrs(job.out), idx, r, o);
 }
 
+// The place in tile order of workgroup b of n. Workgroups go to the 8 XCDs in
+// turn, and an XCD's to its 32 CUs in turn, so in plain order an XCD would get
+// the same columns of every image whose width is a multiple of 8 tiles, and a CU
+// the same tiles of every image of 16 rows of 16 (or twice that, ..): one of
+// them has the dear ones of all. So within each 256 the CU's turn is rotated by a
+// hash of the 256's number and the XCD's by one of the eight's (Fibonacci
+// hashing: the top bits of a product with 2^32 / golden ratio); whatever is left
+// over keeps its order. One run of views of one tree, plain order / rotated / the
+// best persistent variant: 300 of 256x256, caves 256^3 4041 / 2285 / 2305 us,
+// heights 256^3 5645 / 3052 / 3046; 8 of 256x256, caves 512^3 708 / 355 / 344; 300
+// of 64x64, caves 512^3 1026 / 618 / 640; 8 of 1024x1024, caves 512^3 702 / 659 / 723.
+// (The XCD's turn alone: 2771, 4314, 277, 703, 688.) Eight 1080p frames 673 and
+// 670, 24 views of 12 small trees 456 and 442.
+__device__ inline uint32_t tile_place(uint32_t b, uint32_t n) {
+  if (b >= (n & ~255u)) return b;
+  constexpr uint32_t kHash = 0x9E3779B9u;
+  const uint32_t cu = ((b >> 3) + ((b >> 8) * kHash >> 27)) & 31u;
+  const uint32_t eight = (b >> 8 << 5) | cu;
+  return (eight << 3) | ((b + (eight * kHash >> 29)) & 7u);
+}
+
 // One wave per workgroup over one tile, or over 2^rays_log2 of its rays: the
 // hardware hands out the tiles, in order, as slots fall free. The wave's lanes
 // compare the tile with 64 jobs' first tiles at once (in the block of 64 that
@@ -199,7 +220,8 @@ template <int MIN_WAVES, bool LOD>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
 void batch_tile_kernel(const char* __restrict__ table, uint32_t njobs, uint32_t index_offset,
                        uint32_t trees_offset, uint32_t rays_log2) {
-  const uint32_t tile = blockIdx.x >> (6u - rays_log2);
+  const uint32_t place = tile_place(blockIdx.x, gridDim.x);
+  const uint32_t tile = place >> (6u - rays_log2);
   const BatchIndex* index = reinterpret_cast<const BatchIndex*>(table + index_offset);
   uint32_t block = 0, blocks = (njobs + 63u) >> 6;
   while (blocks > 1u) {
@@ -216,7 +238,7 @@ void batch_tile_kernel(const char* __restrict__ table, uint32_t njobs, uint32_t 
   const BatchJob& job = jobs_of(table)[(block << 6) + last];
   const TreeView& tv = reinterpret_cast<const TreeView*>(table + trees_offset)[tree];
   if ((threadIdx.x >> rays_log2) != 0u) return;
-  const uint32_t lane = ((blockIdx.x << rays_log2) & 63u) + threadIdx.x;
+  const uint32_t lane = ((place << rays_log2) & 63u) + threadIdx.x;
   uint32_t local = tile - job.tile_begin;
   if (job.last_first) local = job.tile_count - 1u - local;
   cast_tile<false, LOD, 8, 8>(job, tv, local, lane, nullptr, 0u);
