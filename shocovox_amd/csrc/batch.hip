@@ -541,11 +541,11 @@ hipError_t launch_tiles(const char* table, uint32_t n, uint64_t tiles, bool lod,
 // A job of a per-tile run: like fill_job, but a large ray array keeps no tiles
 // and sets *stream, to run by its own launch (launch_cast_stream). *all counts
 // the tiles of both kinds.
-int fill_job_or_stream(BatchJob& j, const BatchJobIn& in, uint32_t ti, bool per_tile, uint32_t tw,
-                       uint32_t th, uint64_t* tiles, uint64_t* all, bool* lod, bool* stream,
-                       std::string* err) {
+int fill_job_or_stream(BatchJob& j, const BatchJobIn& in, uint32_t ti, bool per_tile, bool alone,
+                       uint32_t tw, uint32_t th, uint64_t* tiles, uint64_t* all, bool* lod,
+                       bool* stream, std::string* err) {
   *stream = per_tile && in.kind == 1 && in.rays &&
-            streams_cast(in.width, in.viewing_distance > 0.0f);
+            streams_cast(in.width, in.viewing_distance > 0.0f, alone);
   bool job_lod = false;
   const int st = fill_job(j, in, ti, tw, th, all, &job_lod, err);
   if (st != SVO_OK) return st;
@@ -773,8 +773,8 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
       ti = it->second;
     }
     bool stream = false;
-    const int st = fill_job_or_stream(out[i], in, ti, v.per_tile, v.tile_w, v.tile_h, &tiles,
-                                      &all_tiles, &any_lod, &stream, err);
+    const int st = fill_job_or_stream(out[i], in, ti, v.per_tile, n == 1, v.tile_w, v.tile_h,
+                                      &tiles, &all_tiles, &any_lod, &stream, err);
     if (st != SVO_OK) return st;
     if (stream) streamed.push_back(i);
   }
@@ -786,7 +786,7 @@ int batch_run(BatchContext* b, const BatchJobIn* jobs, uint32_t n, void* stream,
     for (uint32_t i = 0; i < n; ++i) {
       const uint32_t threshold = cast_order_threshold();
       if (jobs[i].kind != 1 || threshold == 0 || jobs[i].width < threshold ||
-          (v.per_tile && streams_cast(jobs[i].width, jobs[i].viewing_distance > 0.0f)))
+          out[i].tile_count == 0)  // (streamed)
         continue;
       uint32_t* ord = nullptr;
       const int st = order_rays(jobs[i].rays, jobs[i].width, jobs[i].tree->view.size, &ord, s, err);
@@ -960,8 +960,8 @@ int run_static(const svo_job* jobs, uint32_t n, void* stream, std::string* err) 
       trees[ti] = in.tree->view;
     }
     bool stream = false;
-    st = fill_job_or_stream(out[i], in, ti, v.per_tile, v.tile_w, v.tile_h, &tiles, &all_tiles,
-                            &any_lod, &stream, err);
+    st = fill_job_or_stream(out[i], in, ti, v.per_tile, n == 1, v.tile_w, v.tile_h, &tiles,
+                            &all_tiles, &any_lod, &stream, err);
     if (st != SVO_OK) return st;
     if (stream) streamed[nstreamed++] = i;
   }

@@ -1149,9 +1149,19 @@ uint32_t cast_order_threshold() {
 // LOD rays end sooner and gain less, so for them the line is twice as far:
 // 500,009 rays 196 us streamed, 184 one per lane; 1M rays 291 and 295; 3M into
 // a 256^3 heightfield 660 and 999.
-bool streams_cast(uint64_t n, bool lod) {
+// Camera rays are quicker one per lane at any count (4K in 8x8 tiles, caves 512^3:
+// 397 against 624 us; in rows 561 and 878), but the host does not see what the
+// rays are, and random ones lose more (3M into spheres 512^3 1343 against 697).
+// A job among others of a batched run has a line of its own: streamed jobs run one
+// after another, each with a tail in which the chip empties, while the tiles of
+// smaller ones overlap. Streamed / as tiles / the persistent kernel with sorted
+// rays before either, ms: 16 jobs of 400,000 random rays, caves 256^3 3.28 / 2.13 /
+// 3.20; 4 of 900,000 1.18 / 1.24 / 1.86 and spheres 512^3 1.39 / 1.57 / 2.86; 4 of
+// 1.2M 1.42 / 1.61 / 2.54; 4 of 720p camera rays in rows, caves 512^3 0.95 / 0.41 / 0.60.
+bool streams_cast(uint64_t n, bool lod, bool alone) {
   const uint32_t order_from = chosen_order_threshold();
-  return n > uint64_t(kStreamWaves) * (lod ? 128u : 64u) && (order_from == 0u || n < order_from);
+  return n > uint64_t(kStreamWaves) * (lod ? 128u : 64u) && (alone || n >= 1u << 20) &&
+         (order_from == 0u || n < order_from);
 }
 
 int launch_cast_stream(const DeviceTree& t, const float* rays, uint32_t n, float viewing_distance,
@@ -1181,7 +1191,7 @@ int cast_any(const DeviceTree& t, const float* rays, uint32_t n, float viewing_d
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
-  if (streams_cast(n, lod)) {
+  if (streams_cast(n, lod, true)) {
     const int st = launch_cast_stream(t, rays, n, viewing_distance, lod, out, stream, err);
     if (st == SVO_OK) timer.done();
     return st;

@@ -117,9 +117,9 @@ int order_rays(const float* rays, uint32_t n, float tree_size, uint32_t** order,
 // Ray counts from which svo_cast traverses in that order (0: never).
 void set_cast_order_threshold(uint32_t n);
 uint32_t cast_order_threshold();
-// Whether a cast of n rays runs by launch_cast_stream, and that launch (n > 0,
-// rays not NULL)
-bool streams_cast(uint64_t n, bool lod);
+// Whether a cast of n rays runs by launch_cast_stream (`alone`: a call or run of its
+// own, not a job among others), and that launch (n > 0, rays not NULL)
+bool streams_cast(uint64_t n, bool lod, bool alone);
 int launch_cast_stream(const DeviceTree& t, const float* rays, uint32_t n, float viewing_distance,
                        bool lod, const svo_hits& out, void* stream, std::string* err);
 // log2 of the rays a wave takes in a launch over `rays` rays (2 to 6)

@@ -8,7 +8,7 @@ import pytest
 
 import oracle
 from parity import assert_parity, gpu_to_numpy
-from shocovox_amd import DeviceTree, Octree, alloc_hits, workloads as W
+from shocovox_amd import Batch, DeviceTree, Octree, alloc_hits, workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -84,3 +84,46 @@ def test_cast_of_a_frame_takes_about_a_frame(gpu_device):
             v = image[k].reshape(w * h, -1)[order]
             assert torch.equal(v, hits[k].reshape(w * h, -1)), k
         assert cast < 2.5 * frame
+
+
+def test_large_jobs_of_one_run_overlap(gpu_device):
+    """Four 720p arrays in one run: as streamed casts one after another they took
+    what four calls take, as tiles of one launch less than half of it; 0.75 lies
+    between. With a job of more than 2^20 rays, which is streamed, results are
+    those of plain calls too."""
+    import torch
+    size, w, h = 512, 1280, 720
+    dtree = DeviceTree(Octree.scene(2, size, 16, 5))
+    order = torch.from_numpy(_tiles(w, h)).to(gpu_device)
+    arrays = []
+    for i in range(4):
+        vp = W.look_at_viewport((1.4 * size, 0.8 * size, (i - 1.2) * 0.3 * size),
+                                (size / 2, 0.4 * size, size / 2), w, h)
+        rays = oracle.viewport_rays(vp.origin, vp.direction, vp.frustum, vp.fov, w, h)
+        arrays.append(torch.from_numpy(rays).to(gpu_device)[order].contiguous())
+    arrays.append(torch.from_numpy(W.incoherent_rays(size, (1 << 20) + 77, 3)).to(gpu_device))
+    want = [dtree.cast(r, FIELDS) for r in arrays]
+    outs = [alloc_hits(len(r), gpu_device, FIELDS) for r in arrays]
+    for n in (4, 5):
+        for o in outs:
+            for v in o.values():
+                v.fill_(-3)
+        batch = Batch(n)
+        jobs = [Batch.cast_job(dtree, r, o) for r, o in zip(arrays[:n], outs)]
+        times = [], []
+        for _ in range(6):
+            for calls, t in ((lambda: batch.run(jobs), times[0]),
+                             (lambda: [dtree.cast_into(r, len(r), o)
+                                       for r, o in zip(arrays[:n], want)], times[1])):
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                a.record()
+                calls()
+                b.record()
+                torch.cuda.synchronize()
+                t.append(a.elapsed_time(b) * 1e3)
+        run, each = min(times[0]), min(times[1])
+        print(f"{n} jobs: one run {run:.0f} us, {n} casts {each:.0f} us", flush=True)
+        for i in range(n):
+            for k in FIELDS:
+                assert torch.equal(outs[i][k], want[i][k]), (i, k)
+        assert n > 4 or run < 0.75 * each

@@ -19,7 +19,8 @@ F.fake_log.restype = C.c_char_p
 F.fake_news.restype = C.c_ulong
 tree = DeviceTree(Octree.scene(2, 64, 4, 3))
 vp = W.look_at_viewport((90.0, 80.0, -20.0), (32.0, 30.0, 32.0), 40, 24)
-rays = np.zeros((400_000, 6), np.float32)  # (never read here)
+rays = np.zeros(6, np.float32)  # (never read here)
+BIG = (1 << 20) + 77  # rays of a job that runs by its own launch
 def render():
     return N.Job(tree._h, 0, 40, 24, vp.to_c(), None, N.Hits(), 0.0)
 def cast(n):
@@ -54,7 +55,7 @@ def test_static_run_allocates_nothing():
     """svo_batch_run_static makes no allocation on the host either, so it
     cannot run out of memory between two of its launches."""
     fakehip.run(PRELUDE + """
-js = jobs(cast(400_000), render(), cast(400_000), cast(100))
+js = jobs(cast(BIG), render(), cast(BIG), cast(100))
 for _ in range(2):
     before = F.fake_news()
     assert L.svo_batch_run_static(js, 4, S[0]) == 0
@@ -74,7 +75,7 @@ def test_failed_run_keeps_the_work_it_queued(small, kernel, queued):
 small, kernel, queued = {small!r}, {kernel!r}, {queued!r}
 b = C.c_void_p()
 assert L.svo_batch_create(64, C.byref(b)) == 0
-js = jobs(cast(400_000), *[render() for _ in range(1 if small else 60)])
+js = jobs(cast(BIG), *[render() for _ in range(1 if small else 60)])
 def run(s):
     F.fake_clear_log()
     return L.svo_batch_run(b, js, len(js), s)
