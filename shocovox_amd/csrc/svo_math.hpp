@@ -118,9 +118,11 @@ SVO_HD inline uint32_t f2u32(float x) {
 // of extreme exponents (11 instructions a quotient, about 15 a root), for
 // operands known to be far from them; the same values, as both are IEEE 754's.
 //   * rcp_mid: one Newton step from the hardware's estimate. It rounds
-//     correctly for every one of the 2^23 significands (compared on the
-//     device with 1 / b), and nothing in it depends on the exponent while no
-//     operation over- or underflows: |b| in [2^-24, 2^24].
+//     correctly for every one of the 2^23 significands. That is a property of
+//     gfx950's estimates, held by a test over all of them: from estimates one
+//     unit off, 33 significands would round wrong (and 5 in sqrt_mid). Nothing
+//     in it depends on the exponent while no operation over- or underflows:
+//     |b| in [2^-24, 2^24].
 //   * quot_mid(a, b, rcp_mid(b)): Markstein's residual correction (P. Markstein,
 //     IBM J. Res. Dev. 34, 1990). It equals a / b for all 2^46 pairs of
 //     significands (compared on the device), and the residual is exact for
