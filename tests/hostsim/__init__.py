@@ -47,12 +47,14 @@ def ray_lut() -> np.ndarray:
 
 def cast(flat_arrays: dict, rays: np.ndarray, resumable: bool = False,
          max_steps: int = 0, viewing_distance: float | None = None,
-         general: bool = False, regrouped: bool | str = False) -> np.ndarray:
+         general: bool = False, regrouped: bool | str = False,
+         sliced: int = 0) -> np.ndarray:
     """The product traversal on the host: cast_ray, with resumable=True its
     ray_begin / ray_step form, with a viewing distance cast_ray_lod, with
     regrouped=True the while-while form cast_ray_ww (regrouped="nocrawl":
-    that form without the crawl shortcut). As on the device, power-of-two
-    trees take the P2 form unless general=True."""
+    that form without the crawl shortcut), with sliced = 1, 3 or 20 the walk of
+    a streamed cast, bricks in slices of that many cells. As on the device,
+    power-of-two trees take the P2 form unless general=True."""
     a = flat_arrays
     keep = [np.ascontiguousarray(a["nodes"]), np.ascontiguousarray(a["brick_pix"]),
             np.ascontiguousarray(a["brick_occ"]), np.ascontiguousarray(a["colors"]), ray_lut()]
@@ -65,6 +67,8 @@ def cast(flat_arrays: dict, rays: np.ndarray, resumable: bool = False,
     out = np.zeros(len(rays), HIT_DTYPE)
     mode = 2 if viewing_distance is not None else (
         4 if regrouped == "nocrawl" else (3 if regrouped else int(resumable)))
+    if sliced:
+        mode = 10 + 2 * (1, 3, 20).index(sliced) + int(viewing_distance is not None)
     lib().hs_cast(C.byref(t), rays.ctypes.data, len(rays), out.ctypes.data, mode, int(general))
     return out
 

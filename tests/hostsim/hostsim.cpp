@@ -6,6 +6,22 @@
 
 #include "../../shocovox_amd/csrc/traverse.hpp"
 
+// The walk of a streamed cast, alone: bricks in slices of SLICE cells, and the
+// stack iterations that put them off (power-of-two trees).
+template <bool LOD, int SLICE>
+static svo::CastResult cast_sliced(const svo::TreeView& t, svo::V3f o, svo::V3f d,
+                                   float viewing_distance) {
+  svo::RayWalk w;
+  svo::walk_begin<LOD>(t, o, d, w);
+  while (w.end == svo::WALK_RUNS) {
+    if (w.brick == svo::BRICK_DUE)
+      svo::walk_slice<true, SLICE>(t, nullptr, 0u, w);
+    else
+      svo::walk_iterate<LOD, true, true>(t, t.ray_lut, o, nullptr, 0u, viewing_distance, w);
+  }
+  return svo::walk_result<LOD, true>(t, nullptr, 0u, w);
+}
+
 extern "C" {
 
 struct hs_tree {
@@ -20,7 +36,7 @@ struct hs_tree {
   uint32_t color_count;
   uint32_t max_steps;  // 0: the default bound
   uint32_t mips_enabled;
-  float viewing_distance;  // mode 2
+  float viewing_distance;  // modes 2, 11, 13, 15
 };
 
 struct hs_hit {
@@ -36,6 +52,8 @@ struct hs_hit {
 // with t->viewing_distance; mode 3: cast_ray_ww; mode 4: cast_ray_ww without
 // the crawl shortcut. Modes 0, 2 and 3 use the P2 form, as the kernels
 // do, when exact_pow2_sizes holds and `general` is 0, else the general form.
+// Modes 10, 12 and 14: cast_sliced in slices of 1, 3 and 20 cells (P2 trees only);
+// 11, 13, 15: the same at t->viewing_distance.
 void hs_cast(const hs_tree* t, const float* rays, uint64_t n, hs_hit* out, int mode,
              int general) {
   const bool p2 = !general && svo::exact_pow2_sizes(static_cast<uint64_t>(t->size), t->dim);
@@ -57,6 +75,14 @@ void hs_cast(const hs_tree* t, const float* rays, uint64_t n, hs_hit* out, int m
     } else if (mode == 2) {
       c = p2 ? svo::cast_ray_lod<true>(v, v.ray_lut, o, d, t->viewing_distance)
              : svo::cast_ray_lod<false>(v, v.ray_lut, o, d, t->viewing_distance);
+    } else if (mode >= 10) {
+      const float vd = t->viewing_distance;
+      c = mode == 10   ? cast_sliced<false, 1>(v, o, d, vd)
+          : mode == 11 ? cast_sliced<true, 1>(v, o, d, vd)
+          : mode == 12 ? cast_sliced<false, 3>(v, o, d, vd)
+          : mode == 13 ? cast_sliced<true, 3>(v, o, d, vd)
+          : mode == 14 ? cast_sliced<false, 20>(v, o, d, vd)
+                       : cast_sliced<true, 20>(v, o, d, vd);
     } else {
       svo::RayState st;
       if (svo::ray_begin(v, o, d, st)) {
