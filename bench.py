@@ -9,7 +9,7 @@ output per ray: hit, voxel xyz, albedo, distance); the tree is resident in
 HBM before timing starts. Prints one JSON line.
 
 By default a step is one batched launch (svo_batch_run: the 8 render jobs in
-one persistent kernel), whose outputs are checked equal to 8 separate
+one kernel), whose outputs are checked equal to 8 separate
 svo_render launches; `--launch per-frame` times the 8 separate launches
 instead. A single launch ends when its slowest waves end (a few tiles take
 ~10x the mean number of traversal steps), so one launch per frame leaves the
@@ -168,8 +168,7 @@ def batched_bench(args, render_variant: str) -> dict:
     """Batched mode: trees of uneven size (log-uniform 64..max), content of the
     plain heightfield (built bottom-up) or the caves by seed, brick dims
     4/8/16, each with 1-4 viewports of resolution drawn from {128^2, 512^2,
-    720p, 1080p}; all rays in one persistent launch per batch kernel variant
-    (a replayed hipGraph), against one plain render launch per viewport.
+    720p, 1080p}; all rays in one batched run per kernel variant, against one plain render launch per viewport.
     Outputs of the two forms are compared for equality."""
     import torch
 
@@ -617,7 +616,7 @@ def main() -> int:
     ap.add_argument("--served-max-load", type=float, default=4.0,
                     help="upper end of the capacity search, as a fraction of capacity")
     ap.add_argument("--served-kernel-mode", action="store_true",
-                    help="also serve with the persistent kernel for every launch")
+                    help="also serve with the batched kernel for every launch")
     ap.add_argument("--mode", default="render", choices=["render", "copy", "lod"],
                     help="'copy' runs a plain device-to-device copy of known size (for "
                          "calibrating rocprofv3 byte counters); 'lod' times get_by_ray_at_lod "

@@ -303,9 +303,11 @@ typedef struct svo_hits {
 } svo_hits;
 
 /* Octree::get_by_ray for n rays (src/raytracing/raytracing_on_cpu.rs:316-318).
- * rays: device array of n x {origin.xyz, direction.xyz} f32. Large
- * arrays (from about 400,000 rays) are streamed: a wave's lanes take its rays
- * one after another, in no fixed order; each ray's outputs are its own. */
+ * rays: device array of n x {origin.xyz, direction.xyz} f32, directions of unit
+ * length (the reference's cell distances assume it; with other lengths the
+ * results are defined, but for some rays not the reference's). Large arrays
+ * (from about 400,000 rays) are streamed: a wave's lanes take its rays one
+ * after another, in no fixed order; each ray's outputs are its own. */
 int svo_cast(const svo_tree* dtree, const float* rays, uint32_t n, const svo_hits* out,
              void* stream);
 /* No counterpart in the reference (a tuning knob): the ray count from which
@@ -366,11 +368,13 @@ int svo_render_rgba8(const svo_tree* tree, const svo_viewport* viewport, uint32_
 
 /* ---------------------------------------------------------------------- */
 /* Batched mode (no counterpart in the reference, which renders one view    */
-/* per dispatch): many trees, viewports and ray arrays in one persistent    */
-/* launch. Waves pull 64-ray tiles from a device work counter until all     */
-/* tiles of all jobs are done. The launch sequence (job-table upload,       */
-/* counter reset, persistent kernel) is captured once in a hipGraph and     */
-/* replayed for every run.                                                  */
+/* per dispatch): many trees, viewports and ray arrays in one run. By       */
+/* default the job table is uploaded and one launch runs a one-wave         */
+/* workgroup per 64-ray tile of all jobs; a cast job of 2^20 rays or more   */
+/* (or a run's only job, from the size at which svo_cast streams) has a     */
+/* launch of its own after it, as svo_cast's. The persistent variants       */
+/* instead pull tiles from device work counters; their sequence (upload,    */
+/* counter reset, kernel) is a hipGraph replayed for every run.             */
 /* ---------------------------------------------------------------------- */
 
 typedef struct svo_batch svo_batch;
@@ -392,10 +396,10 @@ typedef struct svo_job {
   float viewing_distance;
 } svo_job;
 
-/* A reusable batch context for up to max_jobs jobs; its device buffers and
- * graph live until svo_batch_destroy. Runs on one context execute in call
- * order: a run waits, on its stream, for the context's previous run, and the
- * host blocks only when it would refill the job table of the run two calls
+/* A reusable batch context for up to max_jobs jobs; its device buffers (and a
+ * persistent variant's graph) live until svo_batch_destroy. Runs on one context
+ * execute in call order: a run waits, on its stream, for the context's previous
+ * run, and the host blocks only when it would refill the job table of the run two calls
  * back before that run's copy has finished. Separate contexts may run
  * concurrently on different streams. The context keeps an event recorded on
  * each of its last two runs' streams: such a stream must not be destroyed
@@ -403,8 +407,9 @@ typedef struct svo_job {
  * support waiting on an event last recorded on a destroyed stream). */
 int svo_batch_create(uint32_t max_jobs, svo_batch** out);
 void svo_batch_destroy(svo_batch* batch);
-/* Launches all jobs as one persistent kernel on `stream` (asynchronous). The
- * caller's job array may be reused as soon as the call returns. */
+/* Launches all jobs on `stream` (asynchronous). The caller's job array may be
+ * reused as soon as the call returns. When a launch fails, what was queued
+ * before it still runs, and later runs and svo_batch_destroy wait for it. */
 int svo_batch_run(svo_batch* batch, const svo_job* jobs, uint32_t n, void* stream);
 /* Total 64-ray tiles of the last run. */
 uint64_t svo_batch_tiles(const svo_batch* batch);
@@ -412,7 +417,7 @@ uint64_t svo_batch_tiles(const svo_batch* batch);
  * the reference; for callers that cannot allocate device memory (code under
  * stream capture, tight serving loops, harnesses that forbid hipMalloc). The
  * job table (at most 256 jobs) and the work counters live in a fixed device
- * array of the library (about 64 KiB per device, held until the process
+ * array of the library (about 72 KiB per device, held until the process
  * ends) that every call on a device shares: calls that overlap on one device
  * race, so the caller orders them (one stream, or events). The table reaches
  * the device through kernel arguments, so the call allocates nothing, copies
@@ -421,8 +426,8 @@ uint64_t svo_batch_tiles(const svo_batch* batch);
  * 256 jobs is SVO_INVALID_ARGUMENT. Results equal svo_batch_run's. */
 int svo_batch_run_static(const svo_job* jobs, uint32_t n, void* stream);
 /* Kernel variants of batched launches (no counterpart in the reference):
- * "classic" (one 64-ray tile per work grab, one ray per lane) and lane-refill
- * forms (several tiles per grab; finished lanes start the next rays of the
+ * "auto" (the default, a workgroup per tile) and persistent ones: "classic" (one
+ * 64-ray tile per work grab, one ray per lane), "ww" and lane-refill forms (several tiles per grab; finished lanes start the next rays of the
  * grab). A context keeps the variant selected when it was created; results
  * are identical across variants. */
 int svo_batch_variant_count(void);
@@ -444,11 +449,11 @@ int svo_batch_variant_scratch(int variant, uint32_t* bytes);
 /*    join the next launch; up to max_inflight launches are queued on their */
 /*    own streams.                                                          */
 /*    A launch that would hold a single whole request runs as a plain       */
-/*    render instead (the persistent kernel's set-up buys nothing for one   */
-/*    job), so a lightly loaded loop behaves as mode 1.                     */
+/*    render instead (a batched run's set-up buys nothing for one job), so  */
+/*    a lightly loaded loop behaves as mode 1.                              */
 /*  mode 1, per-request plain launches: each render request is one          */
 /*    svo_render launch, in arrival order, on up to max_inflight streams.  */
-/*  mode 2: mode 0 with the persistent batched kernel for every launch.    */
+/*  mode 2: mode 0 with the batched kernel for every launch.               */
 /* Both modes keep per-tree order: a render sees exactly the edits that     */
 /* arrived before it. Edits run on a pool of host threads (host octree      */
 /* edit, then an asynchronous svo_tree_update on the thread's own stream)   */

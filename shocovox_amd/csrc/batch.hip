@@ -1,9 +1,11 @@
-// Batched mode: every tile of every job in one launch.
+// Batched mode: every tile of every job in one launch, but for large cast jobs,
+// which are streamed by launches of their own after it (streams_cast).
 //
 // A job is a viewport render or a ray-array cast on one resident tree. Its
 // rays are cut into 64-ray tiles (8x8 pixels for renders), numbered
 // contiguously across jobs. The default kernel ("auto", batch_tile_kernel)
-// has one one-wave workgroup per tile, which the hardware hands out in order.
+// has one one-wave workgroup per tile, which the hardware hands out as slots fall
+// free.
 // The persistent variants split the tile space into 8 contiguous chunks, one
 // per XCD (workgroups are dispatched to the 8 XCDs round-robin); each wave
 // takes the next tiles of its XCD's chunk from a device counter and, once that
@@ -211,7 +213,7 @@ __device__ inline uint32_t tile_place(uint32_t b, uint32_t n) {
 }
 
 // One wave per workgroup over one tile, or over 2^rays_log2 of its rays: the
-// hardware hands out the tiles, in order, as slots fall free. The wave's lanes
+// hardware hands out the tiles as slots fall free. The wave's lanes
 // compare the tile with 64 jobs' first tiles at once (in the block of 64 that
 // a binary search leaves), and the tree's index comes with them, so that the
 // job and its tree are read side by side: a wave starts three memory round

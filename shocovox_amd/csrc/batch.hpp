@@ -1,4 +1,4 @@
-// Batched mode: many trees, viewports and ray arrays in one persistent launch.
+// Batched mode: many trees, viewports and ray arrays in one run.
 #pragma once
 
 #include <cstdint>

@@ -67,9 +67,10 @@ __global__ __launch_bounds__(64) void cast_lod_kernel(TreeView t, const float* _
 // the others do not wait for the longest; and each pass is either a walk of the
 // lanes that stand in a brick or a stack-loop iteration of the rest, whichever
 // are more. 3M rays into spheres 512^3 and caves 512^3, kSlice 4 / 8 / 12 / 16 /
-// 24: 923 / 836 / 808 / 790 / 772 and 896 / 841 / 824 / 818 / 826 us; both parts
-// in every pass, kSlice 6: 820 and 893 us. (20 as 16 and 24; kRefill 16 and 32,
-// and lines at a third and two thirds instead of half, measured within 3%.)
+// 20 / 24: 822 / 735 / 712 / 695 / 693 / 681 and 808 / 752 / 733 / 733 / 745 / 737
+// us; 500,000 into caves 256^3 270 / 246 / 239 / 235 / 240 / 240. (Both parts in
+// every pass measured 4 and 8% slower; kRefill 16 and 32, and lines at a third and
+// two thirds instead of half, within 3%.)
 // Groups a grid apart, because neighbouring rays of a camera's array cost alike:
 // with n / grid consecutive rays a wave the launch lasted as long as the waves
 // that had the horizon. 3840x2160 camera rays in rows of pixels / in 8x8 tiles,
@@ -81,8 +82,8 @@ __global__ __launch_bounds__(64) void cast_lod_kernel(TreeView t, const float* _
 // tree's size, in origin: 8x8 pixels of 720p, not 64 in a row) end together, and
 // mixed with the next group's they would only part; after such a group the lanes
 // wait for all 64: 4K in tiles 748 -> 616 us, 720p in tiles 305 -> 254, random
-// rays unchanged. (In rows kNear of 2^-5 measured the same within 15% either way.)
-// The LOD form needs more than the 80 registers that six waves leave it: 24 bytes
+// rays unchanged. (kNear 2^-5: 4K in rows 3% slower to 17% faster, the rest alike.)
+// The LOD form needs more than the 80 registers that six waves leave it: 20 bytes
 // of scratch a lane.
 constexpr int kSlice = 20;
 constexpr uint32_t kRefill = 24;
@@ -569,14 +570,15 @@ bool validate_desc(const svo_tree_desc& d, std::string* err) {
 
 }  // namespace
 
-// log2 of the rays a wave of a plain launch takes: 64 once that makes 2048
-// waves (two per SIMD), fewer, down to 4, for smaller launches. Such a launch
-// lasts as long as its slowest wave, and a wave runs the paths of all its
-// lanes, so a chip with idle SIMDs answers sooner with its rays spread over
-// more waves; beyond about two waves per SIMD the extra instructions cost
-// more. Microseconds with 64 / 32 / 16 / 8 / 4 / 2 rays a wave: 1,009 rays
-// 46 / 39 / 33 / 29 / 28 / 28; 60,000 rays 116 / 96 / 110 / 113 / 123 / 142;
-// a 256x256 frame 75 / 70 / 71 / 71 / 72 / 90; 300,007 rays 152 / 177 / 216.
+// log2 of the rays a wave of a plain launch takes: the fewest, from 4 to 64, that
+// keep the launch within 2048 waves (two per SIMD), so 64 from 65,537 rays on. A
+// small launch lasts as long as its slowest wave, and a wave runs the paths of
+// all its lanes, so a chip with idle SIMDs answers sooner with its rays spread
+// over more waves; beyond about two waves per SIMD the extra instructions cost
+// more. Microseconds with 64 / 32 / 16 / 8 / 4 / 2 rays a wave (calls with their
+// allocations): 1,009 rays 62 / 54 / 52 / 45 / 44 / 42; 60,000 rays 103 / 87 / 92 /
+// 100 / 122 / 132; 100,000 rays 105 / 97 / 110 / 128 / 149 / 183; 300,007 rays 151 /
+// 176 / 210 / 261 / 328 / 434; a 256x256 frame 76 / 71 / 72 / 72 / 84 / 111.
 uint32_t wave_rays_log2(uint64_t rays) {
   uint32_t k = 2;
   while (k < 6 && rays > (uint64_t(2048) << k)) ++k;
@@ -1140,12 +1142,11 @@ uint32_t cast_order_threshold() {
 }
 
 // More rays than lanes run at once: from there on a lane has further rays to
-// take. 3M rays in their own order, streamed against one ray per lane ordered
-// by origin and direction (order.hip; its sort is 0.2 ms): spheres 512^3 0.78
-// against 1.20 ms, caves 512^3 0.82 against 1.37; 1.2M rays, caves 0.41
-// against 0.69; one ray per lane unordered: 1.42, 1.18 and 0.54 ms. Around the
-// line: 300,007 rays 188 streamed, 152 us one per lane; 500,000 rays 214 and
-// 245 us.
+// take. Random rays in their own order, streamed / one per lane / one per lane
+// ordered by origin and direction (order.hip, its sort included), ms: 3M into
+// spheres 512^3 0.70 / 1.33 / 1.12, caves 512^3 0.73 / 1.15; 1.5M into caves 512^3
+// 0.44 / 0.63. Around the line: 300,007 rays 188 streamed, 152 us one per lane;
+// 500,000 into caves 256^3 227 and 265 us.
 // LOD rays end sooner and gain less, so for them the line is twice as far:
 // 500,009 rays 196 us streamed, 184 one per lane; 1M rays 291 and 295; 3M into
 // a 256^3 heightfield 660 and 999.

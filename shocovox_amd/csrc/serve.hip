@@ -470,9 +470,9 @@ int alloc_slot(Slot& sl, uint64_t cap, uint32_t digest_cap, uint32_t batch_jobs)
 // Launches the slot's chunks (already in sl.chunks) and records its event;
 // *single is set when a mode-0 launch ran as one plain render.
 int launch_slot(Session& s, Slot& sl, bool* single) {
-  // Mode 0 runs a launch that holds one whole request as a plain render (the
-  // persistent kernel's job table, counters and graph buy nothing for one
-  // job); mode 2 uses the persistent kernel for every launch.
+  // Mode 0 runs a launch that holds one whole request as a plain render (a
+  // batched run's job table buys nothing for one job); mode 2 uses the batched
+  // kernel for every launch.
   const Chunk& c0 = sl.chunks[0];
   const bool whole = sl.chunks.size() == 1 && c0.first_tile == 0 &&
                      c0.tiles == tiles_of(s.plan[c0.req]);

@@ -364,7 +364,10 @@ SVO_HD inline void dda_step_axes(V3f dir, V3f sig, V3f* p, V3f bmin, float size,
 // on the representable grid of size): for s = +1 both are the once-rounded
 // real value min + size - p; for s = -1 the reference's is p - min exactly
 // and far - p its negation, equal after |.|; for s = NaN every scale factor is
-// NaN and both distances are NaN.
+// NaN and both distances are NaN. The reference's distances assume a direction of
+// unit length. With another length p leaves the cell by any distance, p - min may
+// round, and the two forms part: an impact's last bit for a shorter direction,
+// another cell, or none, for some of the rays of a longer one.
 // Returns the step length m: when m is not NaN, at least one axis steps
 // (fminf returns one of its operands, and m == that operand).
 SVO_HD inline float dda_step_far(V3f dir, V3f* p, V3f far, V3f scale, bool* ax, bool* ay,

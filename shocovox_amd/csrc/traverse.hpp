@@ -3,7 +3,8 @@
 // The control flow and every floating-point operation follow
 // get_by_ray_at_lod with MIP maps disabled (raytracing_on_cpu.rs:325-565),
 // probe_brick (:256-312) and traverse_brick (:156-252), so that one ray takes
-// the same path through the tree, bit for bit, as the reference CPU code:
+// the same path through the tree, bit for bit, as the reference CPU code (the P2
+// form for directions of unit length, see dda_step_far):
 //   * a 4-entry ring stack whose push overwrites the oldest entry and whose
 //     pop past the retained entries restarts from the root after a 0.1 nudge
 //     along the ray (:19-82, :548-562);
@@ -88,7 +89,8 @@ SVO_HD inline uint32_t occ_word(const TreeView& t, uint32_t brick_off, uint32_t 
 // and the POP's a - fmodf(a, b) equals floor(a / b) * b exactly (see
 // pow2_rcp and sub_fmod), so the traversal can be compiled with P2 = true,
 // without the general division and fmodf fallbacks; it is the same
-// arithmetic, bit for bit. (Octree::new checks both powers through f32
+// arithmetic, bit for bit, but for the brick walk of rays whose directions are not
+// of unit length (dda_step_far). (Octree::new checks both powers through f32
 // logarithms, which can admit a non-power at large sizes; such trees take
 // the P2 = false form; the device upload refuses them.)
 SVO_HD inline bool exact_pow2_sizes(uint64_t size, uint64_t dim) {
@@ -490,10 +492,10 @@ SVO_HD __attribute__((always_inline)) inline bool probe_brick(const TreeView& t,
 // the iterations left (tested with a factor of two to spare) the result is
 // known at once. (A NaN component of s makes p leave at the first nudge.)
 // The replay is one chain of adds and compares per ray, thousands long in a
-// large tree: without it a 4K frame of a 1024^3 heightfield takes 0.72 ms
-// instead of 3.04 ms, 24 views of 12 small trees in one batched run 0.71 ms
-// instead of 1.29 ms, and a 720p LOD frame of a 256^3 heightfield 0.25 ms
-// instead of 2.72 ms.
+// large tree: without it a 4K frame of a 1024^3 heightfield took 0.80 ms
+// instead of 2.80 ms, 24 views of 12 small trees in one batched run 0.72 ms
+// instead of 1.17 ms, and a 720p LOD frame of a 256^3 heightfield 0.25 ms
+// instead of 2.69 ms.
 // Not for a leaf root (its brick probe runs on every iteration), nor for
 // MIP-enabled LOD rays unless mip_test_over holds.
 SVO_HD inline CastResult crawl_out_of_root(const TreeView& t, V3f p, V3f d, uint32_t steps,
@@ -575,6 +577,14 @@ struct RingStack {
   }
 };
 
+// lut[i] by a 32-bit byte offset, which the load adds to the base itself (a
+// 64-bit index is added by the vector unit first: 1080p frame 165 -> 163 us,
+// 4K 499 -> 492).
+template <class LutT>
+SVO_HD inline uint64_t lut_word(const LutT* lut, uint32_t i) {
+  return *reinterpret_cast<const LutT*>(reinterpret_cast<const char*>(lut) + (i << 3));
+}
+
 // get_by_ray_at_lod (raytracing_on_cpu.rs:325-565). Without LOD it is
 // get_by_ray (viewing distance f32::MAX, under which the MIP test never
 // passes). `lut` is the RAY_TO_NODE_OCCUPANCY_BITMASK_LUT, wherever the
@@ -606,13 +616,6 @@ struct RingStack {
 // Together a lone ray's iteration takes 0.56 us instead of 0.78, 8 1080p
 // frames in one batched run 0.90 ms instead of 0.96, one of them 0.185 ms
 // instead of 0.208.
-// lut[i] by a 32-bit byte offset, which the load adds to the base itself (a
-// 64-bit index is added by the vector unit first: 1080p frame 165 -> 163 us,
-// 4K 499 -> 492).
-template <class LutT>
-SVO_HD inline uint64_t lut_word(const LutT* lut, uint32_t i) {
-  return *reinterpret_cast<const LutT*>(reinterpret_cast<const char*>(lut) + (i << 3));
-}
 struct RayWalk {
   V3f d, scale, p;
   Cube bounds;

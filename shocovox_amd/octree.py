@@ -630,8 +630,7 @@ def _render_rgba8(tree: "DeviceTree", vp: "Viewport", w: int, h: int, convention
 
 
 class Batch:
-    """Batched mode: many (tree, viewport | rays) jobs in one persistent launch
-    captured in a hipGraph (svo_batch_*)."""
+    """Batched mode: many (tree, viewport | rays) jobs in one run (svo_batch_*)."""
 
     def __init__(self, max_jobs: int):
         h = C.c_void_p()
