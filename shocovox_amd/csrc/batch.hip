@@ -41,6 +41,7 @@
 #include "batch.hpp"
 #include "device_common.hpp"
 #include "handles.hpp"
+#include "launch.hpp"
 #include "refill.hpp"
 
 namespace svo {
@@ -423,8 +424,6 @@ __global__ __launch_bounds__(256) void upload_table_kernel(uint32_t* __restrict_
 }
 
 // Writes `bytes` of a table (a multiple of 4) to the device by upload kernels.
-// (Launch errors are returned by whoever asks for them first, so each helper
-// returns its own, and no kernel is launched on a table that did not arrive.)
 hipError_t upload_table(void* dst, const char* src, size_t bytes, hipStream_t s) {
   const uint32_t words = static_cast<uint32_t>((bytes + 3) / 4);
   for (uint32_t w0 = 0; w0 < words; w0 += kUploadWords) {
@@ -432,9 +431,8 @@ hipError_t upload_table(void* dst, const char* src, size_t bytes, hipStream_t s)
     c.offset_words = w0;
     c.count = std::min(kUploadWords, words - w0);
     std::memcpy(c.words, src + static_cast<size_t>(w0) * 4, static_cast<size_t>(c.count) * 4);
-    hipLaunchKernelGGL(upload_table_kernel, dim3(1), dim3(256), 0, s,
-                       static_cast<uint32_t*>(dst), c);
-    const hipError_t e = hipGetLastError();
+    const hipError_t e =
+        launch(upload_table_kernel, dim3(1), dim3(256), s, static_cast<uint32_t*>(dst), c);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -531,13 +529,8 @@ hipError_t launch_tiles(const char* table, uint32_t n, uint64_t tiles, bool lod,
   const dim3 grid(static_cast<uint32_t>(tiles << (6u - k)));
   const uint32_t index = static_cast<uint32_t>(index_offset_for(n));
   const uint32_t trees = static_cast<uint32_t>(trees_offset_for(n));
-  if (lod)
-    hipLaunchKernelGGL((batch_tile_kernel<6, true>), grid, dim3(64), 0, s, table, n, index, trees,
-                       k);
-  else
-    hipLaunchKernelGGL((batch_tile_kernel<8, false>), grid, dim3(64), 0, s, table, n, index,
-                       trees, k);
-  return hipGetLastError();
+  return launch(lod ? batch_tile_kernel<6, true> : batch_tile_kernel<8, false>, grid, dim3(64), s,
+                table, n, index, trees, k);
 }
 
 // A job of a per-tile run: like fill_job, but a large ray array keeps no tiles
@@ -982,12 +975,10 @@ int run_static(const svo_job* jobs, uint32_t n, void* stream, std::string* err) 
     e = launch_tiles(sd->scratch, n, tiles, any_lod, s);
   } else if (e == hipSuccess) {
     Counter* counters = reinterpret_cast<Counter*>(sd->scratch + kStaticCountersOffset);
-    hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, s, counters);
     const BatchFn fn = any_lod ? v.lod_fn : v.fn;
-    const uint32_t grid = sd->cus * v.groups_per_cu;
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, s, static_cast<const char*>(sd->scratch),
-                       counters);
-    e = hipGetLastError();
+    e = launch(reset_counters_kernel, dim3(1), dim3(64), s, counters);
+    if (e == hipSuccess)
+      e = launch(fn, dim3(sd->cus * v.groups_per_cu), dim3(256), s, sd->scratch, counters);
   }
   if (e != hipSuccess) return hip_fail(e, "svo_batch_run_static launch", err);
   return SVO_OK;

@@ -16,6 +16,7 @@
 #include "device.hpp"
 #include "device_common.hpp"
 #include "flatten.hpp"
+#include "launch.hpp"
 #include "refill.hpp"
 
 namespace svo {
@@ -1024,39 +1025,31 @@ int device_tree_patch(DeviceTree* t, const svo_tree_desc& d, const std::vector<u
   }
   if (!records.empty()) {
     const uint32_t n = static_cast<uint32_t>(records.size());
-    hipLaunchKernelGGL(scatter_records_kernel, dim3((4 * n + 255) / 256), dim3(256), 0, s,
-                       t->nodes, reinterpret_cast<const NodeRec*>(base),
-                       reinterpret_cast<const uint32_t*>(base + o_ridx), n);
-    e = hipGetLastError();
+    e = launch(scatter_records_kernel, dim3((4 * n + 255) / 256), dim3(256), s, t->nodes,
+               reinterpret_cast<const NodeRec*>(base),
+               reinterpret_cast<const uint32_t*>(base + o_ridx), n);
     if (e != hipSuccess) return hip_fail(e, "scatter_records_kernel", err);
   }
   if (bp.n_fills) {
     const uint64_t total = static_cast<uint64_t>(bp.n_fills) * (n3 + words);
-    hipLaunchKernelGGL(fill_slots_kernel, dim3(static_cast<uint32_t>((total + 255) / 256)),
-                       dim3(256), 0, s, t->brick_pix, t->brick_occ,
-                       reinterpret_cast<const uint32_t*>(base + o_fills),
-                       static_cast<uint32_t>(bp.n_fills), n3, words);
-    e = hipGetLastError();
+    e = launch(fill_slots_kernel, dim3(static_cast<uint32_t>((total + 255) / 256)), dim3(256), s,
+               t->brick_pix, t->brick_occ, reinterpret_cast<const uint32_t*>(base + o_fills),
+               static_cast<uint32_t>(bp.n_fills), n3, words);
     if (e != hipSuccess) return hip_fail(e, "fill_slots_kernel", err);
   }
   if (bp.n_whole) {
     const uint64_t total = static_cast<uint64_t>(bp.n_whole) * (n3 + words);
-    hipLaunchKernelGGL(scatter_bricks_kernel, dim3(static_cast<uint32_t>((total + 255) / 256)),
-                       dim3(256), 0, s, t->brick_pix, t->brick_occ,
-                       reinterpret_cast<const uint32_t*>(base + o_bw),
-                       reinterpret_cast<const uint32_t*>(base + o_slots),
-                       static_cast<uint32_t>(bp.n_whole), n3, words);
-    e = hipGetLastError();
+    e = launch(scatter_bricks_kernel, dim3(static_cast<uint32_t>((total + 255) / 256)), dim3(256),
+               s, t->brick_pix, t->brick_occ, reinterpret_cast<const uint32_t*>(base + o_bw),
+               reinterpret_cast<const uint32_t*>(base + o_slots),
+               static_cast<uint32_t>(bp.n_whole), n3, words);
     if (e != hipSuccess) return hip_fail(e, "scatter_bricks_kernel", err);
   }
   if (bp.n_pix + bp.n_occ) {
     const uint32_t n = static_cast<uint32_t>(bp.n_pix + bp.n_occ);
-    hipLaunchKernelGGL(scatter_words_kernel, dim3((n + 255) / 256), dim3(256), 0, s,
-                       t->brick_pix, t->brick_occ,
-                       reinterpret_cast<const uint32_t*>(base + o_writes),
-                       static_cast<uint32_t>(bp.n_pix), static_cast<uint32_t>(bp.n_occ), n3,
-                       words);
-    e = hipGetLastError();
+    e = launch(scatter_words_kernel, dim3((n + 255) / 256), dim3(256), s, t->brick_pix,
+               t->brick_occ, reinterpret_cast<const uint32_t*>(base + o_writes),
+               static_cast<uint32_t>(bp.n_pix), static_cast<uint32_t>(bp.n_occ), n3, words);
     if (e != hipSuccess) return hip_fail(e, "scatter_words_kernel", err);
   }
   if (new_colors) {
@@ -1172,13 +1165,8 @@ int launch_cast_stream(const DeviceTree& t, const float* rays, uint32_t n, float
   // with 82 a wave, 214 with 128)
   const uint32_t groups = (n - 1u) / 64u + 1u;
   const dim3 grid(std::min(kStreamWaves, (groups + 1u) / 2u));
-  if (lod)
-    hipLaunchKernelGGL(cast_stream_kernel<true>, grid, dim3(64), 0, s, t.view, rays, n,
-                       viewing_distance, to_ptrs(out));
-  else
-    hipLaunchKernelGGL(cast_stream_kernel<false>, grid, dim3(64), 0, s, t.view, rays, n,
-                       viewing_distance, to_ptrs(out));
-  const hipError_t e = hipGetLastError();
+  const hipError_t e = launch(lod ? cast_stream_kernel<true> : cast_stream_kernel<false>, grid,
+                              dim3(64), s, t.view, rays, n, viewing_distance, to_ptrs(out));
   return e == hipSuccess ? SVO_OK : hip_fail(e, "cast_stream_kernel launch", err);
 }
 
@@ -1205,13 +1193,11 @@ int cast_any(const DeviceTree& t, const float* rays, uint32_t n, float viewing_d
     if (st != SVO_OK && st != SVO_OUT_OF_DEVICE_MEMORY) return st;
   }
   const uint32_t k = wave_rays_log2(n);
-  if (lod)
-    hipLaunchKernelGGL(cast_lod_kernel, wave_grid(n, k), dim3(64), 0, s, t.view, rays, n,
-                       viewing_distance, order, k, to_ptrs(out));
-  else
-    hipLaunchKernelGGL(cast_kernel, wave_grid(n, k), dim3(64), 0, s, t.view, rays, n, order, k,
-                       to_ptrs(out));
-  const hipError_t e = hipGetLastError();
+  const hipError_t e =
+      lod ? launch(cast_lod_kernel, wave_grid(n, k), dim3(64), s, t.view, rays, n,
+                   viewing_distance, order, k, to_ptrs(out))
+          : launch(cast_kernel, wave_grid(n, k), dim3(64), s, t.view, rays, n, order, k,
+                   to_ptrs(out));
   if (order) (void)hipFreeAsync(order, s);
   if (e != hipSuccess) return hip_fail(e, lod ? "cast_lod_kernel launch" : "cast_kernel launch", err);
   timer.done();
@@ -1237,9 +1223,8 @@ int device_render_lod(const DeviceTree& t, const Camera& cam, uint32_t w, uint32
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
   const Tiles tl = tiles_for(w, h, looks_down(cam, w, h));
-  hipLaunchKernelGGL(frame_lod_kernel, tile_grid(tl), dim3(64), 0, s, t.view, cam, w, h,
-                     viewing_distance, tl, to_ptrs(out));
-  hipError_t e = hipGetLastError();
+  const hipError_t e = launch(frame_lod_kernel, tile_grid(tl), dim3(64), s, t.view, cam, w, h,
+                              viewing_distance, tl, to_ptrs(out));
   if (e != hipSuccess) return hip_fail(e, "frame_lod_kernel launch", err);
   timer.done();
   return SVO_OK;
@@ -1253,9 +1238,8 @@ int device_render(const DeviceTree& t, const Camera& cam, uint32_t w, uint32_t h
   LaunchTimer timer(s);
   if (g_render_variant == kAutoVariant) {
     const Tiles tl = tiles_for(w, h, looks_down(cam, w, h));
-    hipLaunchKernelGGL(frame_kernel, tile_grid(tl), dim3(64), 0, s, t.view, cam, w, h, tl,
-                       to_ptrs(out));
-    const hipError_t e = hipGetLastError();
+    const hipError_t e = launch(frame_kernel, tile_grid(tl), dim3(64), s, t.view, cam, w, h, tl,
+                                to_ptrs(out));
     if (e != hipSuccess) return hip_fail(e, "frame_kernel launch", err);
     timer.done();
     return SVO_OK;
@@ -1273,8 +1257,8 @@ int device_render(const DeviceTree& t, const Camera& cam, uint32_t w, uint32_t h
     const uint64_t waves = (tiles + v.tiles_per_wave - 1) / v.tiles_per_wave;
     grid = dim3(static_cast<uint32_t>((waves + 3) / 4));
   }
-  hipLaunchKernelGGL(v.fn, grid, dim3(v.single_wave_groups ? 64 : 256), 0, s, t.view, cam, w, h, to_ptrs(out));
-  hipError_t e = hipGetLastError();
+  const hipError_t e = launch(v.fn, grid, dim3(v.single_wave_groups ? 64 : 256), s, t.view, cam, w,
+                              h, to_ptrs(out));
   if (e != hipSuccess) return hip_fail(e, "render_kernel launch", err);
   timer.done();
   return SVO_OK;
@@ -1316,13 +1300,8 @@ int device_render_rgba8(const DeviceTree& t, V3f origin, V3f dir, float glass_w,
   hipStream_t s = static_cast<hipStream_t>(stream);
   LaunchTimer timer(s);
   const Tiles tl = tiles_for(w, h, dir.y > 0.0f);  // (row 0 is the top here)
-  if (convention == 0)
-    hipLaunchKernelGGL(shade_kernel<0>, tile_grid(tl), dim3(64), 0, s, t.view, sp, w, h, tl,
-                       out);
-  else
-    hipLaunchKernelGGL(shade_kernel<1>, tile_grid(tl), dim3(64), 0, s, t.view, sp, w, h, tl,
-                       out);
-  const hipError_t e = hipGetLastError();
+  const hipError_t e = launch(convention == 0 ? shade_kernel<0> : shade_kernel<1>, tile_grid(tl),
+                              dim3(64), s, t.view, sp, w, h, tl, out);
   if (e != hipSuccess) return hip_fail(e, "shade_kernel launch", err);
   timer.done();
   return SVO_OK;

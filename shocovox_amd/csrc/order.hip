@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "device.hpp"
+#include "launch.hpp"
 
 namespace svo {
 
@@ -108,10 +109,9 @@ int order_rays(const float* rays, uint32_t n, float tree_size, uint32_t** order,
   if (e == hipSuccess) e = hipMallocAsync(&temp, temp_bytes ? temp_bytes : 1, s);
   if (e == hipSuccess) {
     const uint32_t grid = static_cast<uint32_t>((static_cast<uint64_t>(n) + 255u) / 256u);
-    hipLaunchKernelGGL(ray_keys_kernel, dim3(grid), dim3(256), 0, s, rays, n,
-                       static_cast<float>(kGrid) / tree_size,
-                       static_cast<uint32_t*>(buf[0]), static_cast<uint32_t*>(buf[2]));
-    e = hipGetLastError();
+    e = launch(ray_keys_kernel, dim3(grid), dim3(256), s, rays, n,
+               static_cast<float>(kGrid) / tree_size, static_cast<uint32_t*>(buf[0]),
+               static_cast<uint32_t*>(buf[2]));
   }
   if (e == hipSuccess)
     e = hipcub::DeviceRadixSort::SortPairs(
@@ -124,6 +124,8 @@ int order_rays(const float* rays, uint32_t n, float tree_size, uint32_t** order,
   if (temp) (void)hipFreeAsync(temp, s);
   if (e != hipSuccess) {
     if (buf[3]) (void)hipFreeAsync(buf[3], s);
+    // (without memory the caller goes on unordered: not an error of the thread's)
+    if (e == hipErrorOutOfMemory) (void)hipGetLastError();
     return hip_fail(e, "ray ordering", err);
   }
   *order = static_cast<uint32_t*>(buf[3]);

@@ -36,6 +36,7 @@
 #include "../../include/svo.h"
 #include "batch.hpp"
 #include "handles.hpp"
+#include "launch.hpp"
 
 namespace svo {
 
@@ -556,9 +557,8 @@ int launch_slot(Session& s, Slot& sl, bool* single) {
                                   hipMemcpyHostToDevice, sl.stream);
     if (e != hipSuccess) return hip_err(e, "digest table copy");
     const uint32_t gx = std::min<uint32_t>((max_count + 255) / 256, 512);
-    hipLaunchKernelGGL(digest_kernel, dim3(std::max(gx, 1u), sl.chunks.size()), dim3(256), 0,
-                       sl.stream, sl.d_digest);
-    e = hipGetLastError();
+    e = launch(digest_kernel, dim3(std::max(gx, 1u), sl.chunks.size()), dim3(256), sl.stream,
+               sl.d_digest);
     if (e != hipSuccess) return hip_err(e, "digest_kernel");
   }
   const hipError_t e = hipEventRecord(sl.done, sl.stream);

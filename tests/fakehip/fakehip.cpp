@@ -68,6 +68,8 @@ extern "C" {
 
 void fake_fail_launch(const char* part) { snprintf(g_fail, sizeof(g_fail), "%s", part); }
 const char* fake_log() { return g_log; }
+// Leaves the error of an earlier call behind, as any failed HIP call does.
+void fake_leave_error() { g_last = hipErrorOutOfMemory; }
 void fake_clear_log() { g_log[g_log_len = 0] = 0; }
 unsigned long fake_news() { return g_news; }
 
@@ -150,10 +152,12 @@ hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 // No memory pool: ray ordering finds no memory, and says so in the log.
-hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t*, int) { return hipErrorNotSupported; }
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t*, int) {
+  return g_last = hipErrorNotSupported;
+}
 hipError_t hipMallocAsync(void**, size_t n, hipStream_t s) {
   note("nopool %zu %p\n", n, static_cast<void*>(s));
-  return hipErrorOutOfMemory;
+  return g_last = hipErrorOutOfMemory;
 }
 hipError_t hipFreeAsync(void*, hipStream_t) { return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }

@@ -105,3 +105,41 @@ F.fake_clear_log()
 L.svo_batch_destroy(b)
 assert sum(l[0] == "sync" for l in log()) == 2, log()
 """)
+
+
+def test_an_error_left_by_another_call_is_not_a_launchs():
+    """Any failed HIP call of the thread, the caller's own included, leaves its error
+    for hipGetLastError; launches that succeed do not answer with it."""
+    fakehip.run(PRELUDE + """
+b = C.c_void_p()
+assert L.svo_batch_create(4, C.byref(b)) == 0
+js = jobs(render(), cast(BIG), cast(100))
+hits = C.byref(N.Hits())
+vpc = vp.to_c()
+out = np.zeros(40 * 24, np.uint32)
+calls = dict(
+    batch=lambda: L.svo_batch_run(b, js, 3, S[0]),
+    static=lambda: L.svo_batch_run_static(js, 3, S[0]),
+    cast=lambda: L.svo_cast(tree._h, rays.ctypes.data, 100, hits, S[0]),
+    stream=lambda: L.svo_cast(tree._h, rays.ctypes.data, BIG, hits, S[0]),
+    lod=lambda: L.svo_cast_at_lod(tree._h, rays.ctypes.data, 100, 9.0, hits, S[0]),
+    frame=lambda: L.svo_render(tree._h, C.byref(vpc), 40, 24, hits, S[0]),
+    frame_lod=lambda: L.svo_render_at_lod(tree._h, C.byref(vpc), 40, 24, 9.0, hits, S[0]),
+    shaded=lambda: L.svo_render_rgba8(tree._h, C.byref(vpc), 40, 24, 0, out.ctypes.data, S[0]))
+F.fake_leave_error.restype = None
+wrong = []
+for name, call in calls.items():
+    F.fake_leave_error()
+    if call() != 0:
+        wrong.append((name, error()))
+    assert call() == 0
+assert not wrong, wrong
+# and a launch that fails still says so
+for name, kernel in dict(batch="batch_tile", static="batch_tile", cast="cast_kernel",
+                         stream="cast_stream", lod="cast_lod", frame="frame_kernel",
+                         frame_lod="frame_lod", shaded="shade").items():
+    F.fake_fail_launch(kernel.encode())
+    assert calls[name]() == 7, name
+    F.fake_fail_launch(b"")
+L.svo_batch_destroy(b)
+""")
